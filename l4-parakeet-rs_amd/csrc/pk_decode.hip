@@ -134,11 +134,20 @@ __device__ __forceinline__ float det_exp(float x) {
     q = __builtin_fmaf(q, r, 1.0f);
     return __builtin_ldexpf(q, (int)n);
 }
-__device__ __forceinline__ float det_sigmoid(float v) { return 1.0f / (1.0f + det_exp(-v)); }
+// The IEEE quotient 1 / s for s >= 1 (or NaN).  Below 2^96 it is one Newton
+// step on the hardware reciprocal: compared with the division for every
+// mantissa (the step scales with powers of two), no bit differs; three
+// instructions instead of the division's ten.
+__device__ __forceinline__ float rcp_rn(float s) {
+    if (__builtin_amdgcn_ballot_w64(!(s < 0x1p96f)) != 0) return 1.0f / s;
+    const float r = __builtin_amdgcn_rcpf(s);
+    return __builtin_fmaf(__builtin_fmaf(-r, s, 1.0f), r, r);
+}
+__device__ __forceinline__ float det_sigmoid(float v) { return rcp_rn(1.0f + det_exp(-v)); }
 // tanh(x) = sign(x) (1 - e^-2|x|) / (1 + e^-2|x|): absolute error ~1e-7.
 __device__ __forceinline__ float det_tanh(float v) {
     const float t = det_exp(-2.0f * __builtin_fabsf(v));
-    return __builtin_copysignf((1.0f - t) / (1.0f + t), v);
+    return __builtin_copysignf(div_rn(1.0f - t, 1.0f + t, rcp_rn(1.0f + t)), v);
 }
 
 // decoder.cu:116-129 lstm_cell with the transcendental functions above; the
@@ -742,6 +751,679 @@ __global__ __launch_bounds__(kDecThreads, 1) void tdt_decode_kernel(DecodeArgs p
     }
 }
 
+// ---- the model's decoder width: 64 workgroups ------------------------------------
+//
+// At H = 640 the decode is a chain of small exchanges, not of arithmetic: every
+// emitted token needs the layer-1 output, the prediction and the joint's best
+// keys from all workgroups in turn.  Measured on an MI355X, one exchange (publish,
+// poll until everybody's words are there) takes 2.74 us among 160 workgroups,
+// 1.65 among 128, 1.31 among 64 and 1.13 among 16, on one XCD or on eight; but
+// 3.3 us among 64 when every wave stores its own word instead of one wave a
+// workgroup's ten in one 80-byte store, 3.7 with a second small store beside it.
+// So this form uses 64 workgroups of ten waves (one hidden unit a wave, as above):
+//  - What the others need travels in the exchange itself: a published word is
+//    {fp32 value, epoch tag}, one contiguous store per workgroup, and thread t
+//    of every workgroup polls word t, so there is no store-then-flag wait and no
+//    load after the exchange.
+//  - x = relu(enc + pred) of the window's frames is formed once per workgroup,
+//    by thread k for feature k, and shared through LDS; a wave then scores four
+//    joint rows against four frames (eight waves: 16 rows x 8 frames), rows
+//    past 1024 go one to a workgroup and their eight frames to waves 8 and 9.
+//  - An eleventh wave keeps the next 32 encoder rows in LDS, so that no poll
+//    waits behind a load from HBM, and stores the layer-0 sums.
+//  - Sums over the wave's 64 lanes keep the association of add_level's levels
+//    1, 2, 4, ..., 32, but N sums reduced together halve their number at each
+//    level (lanes_sum): 16 sums take about 60 instructions instead of 200.
+// Every sum has the association of tdt_decode_kernel's, so the tokens are the same.
+// 7500 frames, 2333 tokens, INT8 joint, long form: 41.1 -> 19.6 ms (8.2 us a
+// token: three exchanges of 0.8 us, 0.9 us for layer 0 and 0.8 us each for the
+// joint and for layer 1); on a slower box 69.3 -> 31.7 ms.  93 frames, fp16
+// form: 1003 -> 600 us on the latter.
+constexpr int k640H = 640, k640KP = 5, k640Blocks = 64, k640Waves = 10, k640Rows = 16;
+constexpr int k640Threads = 64 * (k640Waves + 1);  // and a wave that loads the encoder rows
+constexpr int k640Ring = 32;                        // encoder rows kept in LDS
+static_assert(k640Ring >= kWin + kWin - 1 + 7, "the next round's window is loaded before its round");
+constexpr int k640Outputs = k640Blocks * (k640Rows + 1);
+// u32 offsets in the workspace, around the prediction at kDecState + 8 H
+constexpr int k640Joint = 8;                                         // u64 [2][64][kWin]
+constexpr int k640Max = k640Joint + 2 * kWin * k640Blocks * 2;     // u64 [64][3]
+constexpr int k640Pred = k640Max + k640Blocks * 3 * 2;             // u64 [2][H]
+constexpr int k640Out = kDecState + 8 * k640H;                      // float [H]: the last prediction
+constexpr int k640H1 = k640Out + k640H;                            // u64 [2][H]
+constexpr int k640H0 = k640H1 + 4 * k640H;                         // u64 [2][H] (fp16 form)
+constexpr int k640R0 = k640H0 + 4 * k640H;                         // u64 [H][4] (long form)
+static_assert(k640Pred + 4 * k640H <= k640Out, "workspace layout");
+static_assert(k640R0 + 8 * k640H <= kDecState + 9 * k640H + kDecExtWords + 8 * k640H, "workspace size");
+
+// 4 bytes global -> LDS per lane: lane l writes LDS bytes [lds_addr + 4 l, + 4).
+// lds_addr must be wave-uniform; one wait state between the M0 write and the
+// load that reads it.
+__device__ __forceinline__ void dma4(const void* src, uint32_t lds_addr) {
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(src),
+                 "s"(__builtin_amdgcn_readfirstlane(lds_addr))
+                 : "memory", "m0");
+}
+
+// v[l ^ 4] and v[l ^ 8] of a row of 16 lanes, whatever the lanes hold.
+__device__ __forceinline__ float xor4(float v) {
+    const int s = __float_as_int(v);
+    const int t = __builtin_amdgcn_update_dpp(s, s, 0x104, 0xf, 0x5, false);            // row_shl:4 into quads 0 and 2
+    return __int_as_float(__builtin_amdgcn_update_dpp(t, s, 0x114, 0xf, 0xa, false));   // row_shr:4 into quads 1 and 3
+}
+__device__ __forceinline__ float xor8(float v) { return dpp_f<0x128>(v); }  // row_ror:8
+
+// Wave sums of N values (4 or 16), lane l receiving that of value l mod N: at
+// the first log2(N) levels the two lanes of a pair each keep one of two values
+// and hand the other over.  Every sum is that of add_level's levels 1 .. 32.
+template <int N> __device__ __forceinline__ float lanes_sum(float (&v)[N], int lane) {
+#pragma unroll
+    for (int i = 0; i < N / 2; ++i) {
+        const bool b = lane & 1;
+        v[i] = (b ? v[2 * i + 1] : v[2 * i]) + dpp_f<0xB1>(b ? v[2 * i] : v[2 * i + 1]);
+    }
+#pragma unroll
+    for (int i = 0; i < N / 4; ++i) {
+        const bool b = lane & 2;
+        v[i] = (b ? v[2 * i + 1] : v[2 * i]) + dpp_f<0x4E>(b ? v[2 * i] : v[2 * i + 1]);
+    }
+    float s;
+    if constexpr (N == 16) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const bool b = lane & 4;
+            v[i] = (b ? v[2 * i + 1] : v[2 * i]) + xor4(b ? v[2 * i] : v[2 * i + 1]);
+        }
+        const bool b = lane & 8;
+        s = (b ? v[1] : v[0]) + xor8(b ? v[0] : v[1]);
+    } else {
+        s = v[0] + xor4(v[0]);
+        s = s + xor8(s);
+    }
+    return add_level(add_level(s, 16), 32);
+}
+
+// Integer wave sums (exact in any order).  Four values: lane l receives value
+// 2 (l / 32) + (l / 16) % 2.
+__device__ __forceinline__ int swap_add32(int a, int b) {  // lanes < 32: a's sums over l, l ^ 32; the others b's
+    const auto q = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+    return (int)q[0] + (int)q[1];
+}
+__device__ __forceinline__ int swap_add16(int a, int b) {  // even rows of 16: a's sums over l, l ^ 16; odd rows b's
+    const auto q = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+    return (int)q[0] + (int)q[1];
+}
+__device__ __forceinline__ int row_isum4(const int (&v)[4]) { return swap_add16(swap_add32(v[0], v[2]), swap_add32(v[1], v[3])); }
+__device__ __forceinline__ int half_row_isum(int s) { return add_level(add_level(add_level(s, 1), 2), 4); }
+
+// The greedy rules (decoder.cu:773-783) over a round's window, from its
+// decisions (token | duration << 16 in lanes 0 .. kWin - 1): blank decisions
+// keep the prediction, so later frames' decisions in the window stand until a
+// token or the window's end.  emit(token) is called for a token.
+struct GreedyState {
+    int frame = 0, symbols = 0, steps = 0;
+};
+template <typename Emit>
+__device__ __forceinline__ void greedy_round(GreedyState& g, int decided, int blank, int frames, int max_symbols, Emit&& emit) {
+    const int f0 = g.frame;
+    int c = 0;
+    while (true) {
+        const int d = __builtin_amdgcn_readlane(decided, c);
+        const int token = d & 0xffff, dur = d >> 16;
+        ++g.steps;
+        if (token != blank) emit(token);
+        ++g.symbols;
+        g.frame += dur;
+        if (dur != 0 || g.symbols == max_symbols) {
+            if (dur == 0) ++g.frame;
+            g.symbols = 0;
+        }
+        if (token != blank || g.frame >= frames) return;
+        c = g.frame - f0;
+        if (c >= kWin) return;
+    }
+}
+
+template <bool kInt8, bool kLong>
+__global__ __launch_bounds__(k640Threads) void tdt_decode_640_kernel(DecodeArgs p) {
+    constexpr int H = k640H, KP = k640KP, KD = 3, NB = k640Blocks;
+    typedef unsigned long long u64;
+    __shared__ __attribute__((aligned(16))) uint16_t enc_s[k640Ring][H];  // encoder rows frame .. frame + k640Ring - 1
+    __shared__ float x_s[kWin][H];                       // relu(enc + pred) of the window's frames
+    __shared__ float h_s[kLong ? 1 : 4][H];              // long: layer 1's output; fp16: [bank][layer]
+    __shared__ uint32_t q_s[2][kLong ? H / 4 : 1];       // long: the INT8 outputs of layers 0 and 1
+    __shared__ u64 key_s[kWin][8];                       // best key of four rows each, entry 4: of the row past 1024
+    __shared__ __attribute__((aligned(16))) float dur_s[kWin][8];
+    __shared__ u64 win_s[8][kWin];                       // best key of the eight workgroups a wave polled
+    __shared__ float out_s[2][k640Waves];               // this workgroup's values of an exchange
+    __shared__ int r0_s[kLong ? k640Waves * 4 : 1];     // and its layer-0 sums
+    __shared__ int win_dur[kWin];
+    __shared__ float red_s[k640Waves * 3];
+    __shared__ int stop_s;
+    const int blk = blockIdx.x;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int u = min(blk * k640Waves + wave, H - 1);  // this wave's hidden unit
+    const int T = p.token_outputs, D = p.durations, blank = T - 1;
+    auto words = [&](int off) { return (u64*)(p.ws + off); };
+
+    if (tid == 0) stop_s = 0;
+    if (tid < kWin * 8) {
+        key_s[tid >> 3][tid & 7] = 0ull;
+        dur_s[tid >> 3][tid & 7] = 0.0f;
+    }
+    __syncthreads();
+
+    auto publish = [&](u64* w, uint32_t v, uint32_t tag) {
+        __hip_atomic_store(w, ((u64)v << 32) | tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    // the workgroup's ten values, gathered in out_s[i], to their words
+    auto publish_out = [&](u64* w, int i, uint32_t tag) {
+        __syncthreads();
+        if (wave == 0 && lane < k640Waves) publish(w + blk * k640Waves + lane, __float_as_uint(out_s[i][lane]), tag);
+    };
+    // The wave polls its lanes' words until all carry the tag.  Bounded: after
+    // kDecSpinLimit polls, or once another workgroup gave up, the wave sets
+    // stop_s, which the workgroup checks behind its next barrier.
+    auto poll = [&](const u64* w, uint32_t mask, uint32_t tag) -> u64 {
+        u64 v;
+        uint32_t spins = 0;
+        while (true) {
+            v = __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (__builtin_amdgcn_ballot_w64(((uint32_t)v & mask) != tag) == 0) break;
+            if ((++spins & 63) == 0 && (spins > kDecSpinLimit || ld_word(&p.ws[0]) != 0u)) {
+                st_word(&p.ws[0], 1u);
+                stop_s = 1;
+                break;
+            }
+        }
+        return v;
+    };
+    // Four words a lane at once, with the tag the first poll usually finds.
+    auto poll4 = [&](const u64* w, uint32_t tag, int (&v)[4]) {
+        u64 q[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) q[i] = __hip_atomic_load(w + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            if (__builtin_amdgcn_ballot_w64((uint32_t)q[i] != tag) != 0) q[i] = poll(w + i, 0xffffffffu, tag);
+            v[i] = (int)(q[i] >> 32);
+        }
+    };
+    auto value = [](u64 w) { return __uint_as_float((uint32_t)(w >> 32)); };
+
+    // The round's decisions from the waves' keys, in every wave: lanes c, c + 8,
+    // ... hold window frame c's, token | duration << 16.  The largest key is the
+    // best token; workgroup 0's carries the duration.
+    auto max8 = [](u64 v) {  // over lanes l, l ^ 8, l ^ 16, ...
+        const u64 o = ((u64)(uint32_t)dpp_mov<0x128>((int)(v >> 32)) << 32) | (uint32_t)dpp_mov<0x128>((int)(uint32_t)v);
+        return max_level(max_level(o > v ? o : v, 16), 32);
+    };
+    auto decisions = [&]() {
+        const u64 b = max8(win_s[lane >> 3][lane & 7]);
+        return (int)(0xffffu - ((uint32_t)b >> 16)) | (win_dur[lane & 7] << 16);
+    };
+
+    // ---- wave 10: the encoder rows ---------------------------------------------
+    // It follows the decisions and keeps the ring full with direct-to-LDS loads,
+    // a round ahead of their use (a round advances at most kWin - 1 + 7 frames),
+    // so that no exchange waits behind a load from HBM.  It meets every barrier
+    // of the other waves (their loop below): at the start, and per update and
+    // per round.
+    if (wave == k640Waves) {
+        const uint32_t ring = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint16_t*)&enc_s[0][0];
+        int loaded = 0;
+        auto load_to = [&](int end) {
+            for (; loaded < min(end, p.frames); ++loaded)
+#pragma unroll
+                for (int j = 0; j < KP; ++j)
+                    dma4(p.enc + (size_t)loaded * p.enc_stride + 2 * lane + 128 * j,
+                         ring + (uint32_t)(loaded & (k640Ring - 1)) * (2 * H) + 256 * j);
+        };
+        load_to(k640Ring);
+        if constexpr (kLong) __syncthreads();  // the maxima
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        GreedyState g;
+        bool valid = false;
+        uint32_t updates = 0;
+        while (g.frame < p.frames) {
+            if (!valid) {
+                ++updates;
+                __syncthreads();
+                __syncthreads();
+                if constexpr (!kLong) {
+                    if (stop_s) return;
+                    __syncthreads();
+                }
+                __syncthreads();
+                if (stop_s) return;
+                // one bank of layer-0 sums: every workgroup has taken part in the
+                // layer-1 exchange just polled, so it has read the last update's
+                if constexpr (kLong)
+                    if (lane < 4 * k640Waves)
+                        publish(words(k640R0) + blk * (4 * k640Waves) + lane, (uint32_t)r0_s[lane], updates);
+                __syncthreads();
+                valid = true;
+            }
+            __syncthreads();
+            if (stop_s) return;
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __syncthreads();
+            __syncthreads();
+            if (stop_s) return;
+            greedy_round(g, decisions(), blank, p.frames, p.max_symbols, [&](int) { valid = false; });
+            load_to(g.frame + k640Ring);
+        }
+        return;
+    }
+
+    // ---- weights into registers ------------------------------------------------
+    uint32_t wih[kLong ? 1 : 2][4][KP], whh[kLong ? 1 : 2][4][KP], wpj[KP];
+    uint32_t qw[kLong ? 3 : 1][4][KD];  // long form: INT8 rows of W_hh0, W_hh1, W_ih1
+    float cq[3] = {1.0f, 1.0f, 1.0f};   // and their scale / 127
+    // the gate whose sum this lane holds after a reduction, and its bias
+    const int gate = kLong ? lane >> 4 : lane & 3;
+    const float bias1 = p.b_ih[1][gate * H + u] + p.b_hh[1][gate * H + u];
+    const float bias0 = p.b_ih[0][gate * H + u] + p.b_hh[0][gate * H + u];
+    if constexpr (!kLong) {
+#pragma unroll
+        for (int l = 0; l < 2; ++l)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const size_t row = (size_t)(g * H + u) * H + 2 * lane;
+#pragma unroll
+                for (int j = 0; j < KP; ++j) {
+                    wih[l][g][j] = *(const uint32_t*)(p.w_ih[l] + row + 128 * j);
+                    whh[l][g][j] = *(const uint32_t*)(p.w_hh[l] + row + 128 * j);
+                }
+            }
+        for (int i = tid; i < 4 * H; i += H) (&h_s[0][0])[i] = 0.0f;
+    } else {
+        // per-tensor maxima over the whole grid, as above
+        const uint16_t* src[3] = {p.w_hh[0], p.w_hh[1], p.w_ih[1]};
+        constexpr int n8 = H * H / 2;  // 16-byte chunks of a [4H x H] fp16 matrix
+        float mx[3];
+#pragma unroll
+        for (int m = 0; m < 3; ++m) {
+            float a = 0.0f;
+            for (int i = blk * H + tid; i < n8; i += NB * H) {
+                const uint4 v = ((const uint4*)src[m])[i];
+                const uint32_t w4[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    a = __builtin_fmaxf(a, __builtin_fmaxf(__builtin_fabsf(lo16(w4[e])), __builtin_fabsf(hi16(w4[e]))));
+            }
+            mx[m] = wave_max(a);
+        }
+        if (lane == 0)
+#pragma unroll
+            for (int m = 0; m < 3; ++m) red_s[wave * 3 + m] = mx[m];
+        __syncthreads();
+        if (tid < 3) {
+            float a = red_s[tid];
+            for (int i = 1; i < k640Waves; ++i) a = __builtin_fmaxf(a, red_s[i * 3 + tid]);
+            publish(words(k640Max) + blk * 3 + tid, __float_as_uint(a), 1u);
+        }
+        float scale[3];
+#pragma unroll
+        for (int m = 0; m < 3; ++m) {
+            const float t = wave_max(value(poll(words(k640Max) + lane * 3 + m, 0xffffffffu, 1u)));
+            scale[m] = t > 0.0f ? t / 127.0f : 1.0f;
+            cq[m] = scale[m] / 127.0f;
+        }
+#pragma unroll
+        for (int m = 0; m < 3; ++m)
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+#pragma unroll
+                for (int j = 0; j < KD; ++j) {
+                    const int k = 4 * lane + 256 * j;
+                    uint32_t word = 0;
+                    if (k < H) {
+                        const uint2 hv = *(const uint2*)(src[m] + (size_t)(g * H + u) * H + k);
+                        word = (uint32_t)(uint8_t)quant_i8(lo16(hv.x) / scale[m]) | ((uint32_t)(uint8_t)quant_i8(hi16(hv.x) / scale[m]) << 8) |
+                               ((uint32_t)(uint8_t)quant_i8(lo16(hv.y) / scale[m]) << 16) |
+                               ((uint32_t)(uint8_t)quant_i8(hi16(hv.y) / scale[m]) << 24);
+                    }
+                    qw[m][g][j] = word;
+                }
+    }
+#pragma unroll
+    for (int j = 0; j < KP; ++j) wpj[j] = *(const uint32_t*)(p.w_proj + (size_t)u * H + 2 * lane + 128 * j);
+    const float bpj = p.b_proj[u];
+    // joint rows: waves 0 .. 7 own rows 4 (wave % 4) .. + 3 of the workgroup's 16
+    // for frames 4 (wave / 4) .. + 3 of the window, waves 8 and 9 the row past
+    // 1024 if there is one.  Logical order: the duration rows first, so
+    // workgroup 0 holds them all.
+    const bool extra = wave >= 8;
+    const int fh = extra ? wave - 8 : wave >> 2;
+    auto joint_id = [&](int r) {
+        const int i = extra ? (r == 0 ? NB * k640Rows + blk : T + D) : blk * k640Rows + 4 * (wave & 3) + r;
+        return i < D ? T + i : (i < T + D ? i - D : -1);
+    };
+    // The long form keeps INT8 weights as fp32 values, the fp16 form, short of
+    // registers, four to a dword; fp16 weights stay pairs.
+    constexpr bool kWide = kInt8 && kLong;
+    constexpr int JW = kWide ? 2 * KP : (kInt8 ? (KP + 1) / 2 : KP);
+    uint32_t wj[4][JW];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int id = joint_id(r), row = id < 0 ? p.outputs - 1 : id;
+#pragma unroll
+        for (int j = 0; j < KP; ++j) {
+            const size_t at = (size_t)row * H + 2 * lane + 128 * j;
+            if constexpr (kInt8) {
+                const uint32_t w = *(const uint16_t*)((const int8_t*)p.w_joint + at);
+                if constexpr (kWide) {
+                    wj[r][2 * j] = __float_as_uint((float)(int8_t)(w & 0xffu));
+                    wj[r][2 * j + 1] = __float_as_uint((float)(int8_t)((w >> 8) & 0xffu));
+                } else {
+                    wj[r][j / 2] = (j & 1) ? wj[r][j / 2] | (w << 16) : w;
+                }
+            } else {
+                wj[r][j] = *(const uint32_t*)((const uint16_t*)p.w_joint + at);
+            }
+        }
+    }
+    // the row whose sums this lane holds after a reduction
+    const int my_id = joint_id(extra ? 0 : lane & 3);
+    const int my_row = my_id < 0 ? p.outputs - 1 : my_id;
+    const float my_scale = kInt8 ? p.joint_scales[my_row] : 1.0f, my_bias = p.b_joint[my_row];
+
+    // long form: thread t evaluates layer 0 of unit t in every workgroup
+    float b0[4], c0c = 0.0f, c0n = 0.0f;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) b0[g] = kLong ? p.b_ih[0][g * H + tid] + p.b_hh[0][g * H + tid] : 0.0f;
+
+    __syncthreads();
+    GreedyState g;
+    int last = blank, count = 0, alt = 0;
+    uint32_t updates = 0, rounds = 0;
+    bool emitted = false, valid = false, failed = false;
+    float pv = 0.0f;                                                // prediction value of feature tid
+    int rs = 0, rs_next = 0;                                        // long: layer 1's recurrent sum of this lane's gate
+    float c_cur[2] = {0.0f, 0.0f}, c_new[2] = {0.0f, 0.0f};         // cell states of unit u
+    while (g.frame < p.frames) {
+        // Packed weights are unpacked where they are used: without this the
+        // compiler hoists the conversions out of the loop and spills.
+        auto keep = [](uint32_t& w) { asm volatile("" : "+v"(w)); };
+#pragma unroll
+        for (int j = 0; j < KP; ++j) {
+            keep(wpj[j]);
+            if constexpr (!kLong)
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    keep(wih[i >> 2][i & 3][j]);
+                    keep(whh[i >> 2][i & 3][j]);
+                }
+        }
+        if constexpr (!kWide)
+#pragma unroll
+            for (int i = 0; i < 4 * JW; ++i) keep(wj[i / JW][i % JW]);
+        if (!valid) {
+            const uint32_t tag = ++updates;
+            const int par = (int)(tag & 1u);
+            u64* h1w = words(k640H1) + par * H;
+            u64* pw = words(k640Pred) + par * H;
+            if constexpr (!kLong) {
+                // ---- two LSTM layers on the last token's embedding (zeros before any)
+                u64* h0w = words(k640H0) + par * H;
+#pragma unroll
+                for (int l = 0; l < 2; ++l) {
+                    float s[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                    for (int j = 0; j < KP; ++j) {
+                        const int k = 2 * lane + 128 * j;
+                        float2 x = make_float2(0.0f, 0.0f);
+                        if (l == 0) {
+                            if (emitted) {
+                                const uint32_t e = *(const uint32_t*)(p.emb + (size_t)last * H + k);
+                                x = make_float2(lo16(e), hi16(e));
+                            }
+                        } else {
+                            x = *(const float2*)&h_s[(alt ^ 1) * 2][k];  // this update's layer-0 output
+                        }
+                        const float2 hv = *(const float2*)&h_s[alt * 2 + l][k];
+#pragma unroll
+                        for (int g = 0; g < 4; ++g) {
+                            s[g] = __builtin_fmaf(lo16(wih[l][g][j]), x.x, s[g]);
+                            s[g] = __builtin_fmaf(hi16(wih[l][g][j]), x.y, s[g]);
+                            s[g] = __builtin_fmaf(lo16(whh[l][g][j]), hv.x, s[g]);
+                            s[g] = __builtin_fmaf(hi16(whh[l][g][j]), hv.y, s[g]);
+                        }
+                    }
+                    const float v = lanes_sum(s, lane) + (l == 0 ? bias0 : bias1);
+                    const int act = __float_as_int(gate == 2 ? tanhf(v) : sigmoid(v));
+                    const float ig = __int_as_float(__builtin_amdgcn_readlane(act, 0)), fg = __int_as_float(__builtin_amdgcn_readlane(act, 1));
+                    const float cg = __int_as_float(__builtin_amdgcn_readlane(act, 2)), og = __int_as_float(__builtin_amdgcn_readlane(act, 3));
+                    c_new[l] = fg * c_cur[l] + ig * cg;
+                    const float h = og * tanhf(c_new[l]);
+                    u64* w = l == 0 ? h0w : h1w;
+                    if (lane == 0) out_s[0][wave] = h;
+                    publish_out(w, 0, tag);
+                    h_s[(alt ^ 1) * 2 + l][tid] = value(poll(w + tid, 0xffffffffu, tag));
+                    __syncthreads();
+                    if (stop_s) failed = true;
+                    if (failed) break;
+                }
+                if (failed) break;
+            } else {
+                // ---- layer 0 of unit tid: recurrent sums of the committed state +
+                // bias + the token's table row (decoder.cu:619-648)
+                float s[4];
+                uint16_t tv[4] = {0, 0, 0, 0};
+                int r0[4] = {0, 0, 0, 0};
+                if (emitted) {
+#pragma unroll
+                    for (int g = 0; g < 4; ++g) tv[g] = p.table[(size_t)last * 4 * H + g * H + tid];
+                    // published by the last update after its layer-1 exchange; overwritten
+                    // after this update's, which waits for this workgroup
+                    poll4(words(k640R0) + tid * 4, tag - 1, r0);
+                }
+#pragma unroll
+                for (int g = 0; g < 4; ++g) s[g] = __builtin_fmaf((float)r0[g], cq[0], b0[g]) + h2f(tv[g]);
+                float h0;
+                lstm_cell(s, c0c, c0n, h0);
+                ((uint8_t*)q_s[0])[tid] = (uint8_t)quant_i8(h0 * 127.0f);
+                __syncthreads();
+                // ---- layer 1: its recurrent sums + W_ih1 x the new INT8 layer-0
+                // output (decoder.cu:650-670), and the layer-0 recurrent sums of the
+                // new candidate state, which go out for the update after it is committed
+                uint32_t x[KD];
+#pragma unroll
+                for (int j = 0; j < KD; ++j) x[j] = 4 * lane + 256 * j < H ? q_s[0][lane + 64 * j] : 0u;
+                int in[4], r0n[4];
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    int a = 0, d = 0;
+#pragma unroll
+                    for (int j = 0; j < KD; ++j) {
+                        a = __builtin_amdgcn_sdot4((int)qw[2][g][j], (int)x[j], a, false);
+                        d = __builtin_amdgcn_sdot4((int)qw[0][g][j], (int)x[j], d, false);
+                    }
+                    in[g] = a;
+                    r0n[g] = d;
+                }
+                const int ia = row_isum4(in), ra = row_isum4(r0n);
+                const bool hi = lane & 8;  // lanes 8 .. 15 of a row take the layer-0 sum, the others layer 1's
+                const int sum = half_row_isum((hi ? ra : ia) + dpp_mov<0x128>(hi ? ia : ra));
+                if ((lane & 15) == 8) r0_s[wave * 4 + gate] = sum;  // wave 10 publishes them
+                const float v = __builtin_fmaf((float)sum, cq[2], __builtin_fmaf((float)rs, cq[1], bias1));
+                // det_sigmoid, or det_tanh for the cell gate, with one exponential
+                const float e = det_exp(gate == 2 ? -2.0f * __builtin_fabsf(v) : -v);
+                const float r = rcp_rn(1.0f + e);
+                const int act = __float_as_int(gate == 2 ? __builtin_copysignf(div_rn(1.0f - e, 1.0f + e, r), v) : r);
+                const float ig = __int_as_float(__builtin_amdgcn_readlane(act, 0)), fg = __int_as_float(__builtin_amdgcn_readlane(act, 16));
+                const float cg = __int_as_float(__builtin_amdgcn_readlane(act, 32)), og = __int_as_float(__builtin_amdgcn_readlane(act, 48));
+                c_new[1] = __builtin_fmaf(fg, c_cur[1], ig * cg);
+                const float hn = og * det_tanh(c_new[1]);
+                if (lane == 0) out_s[0][wave] = hn;
+                publish_out(h1w, 0, tag);
+                const float h1 = value(poll(h1w + tid, 0xffffffffu, tag));
+                h_s[0][tid] = h1;
+                ((uint8_t*)q_s[1])[tid] = (uint8_t)quant_i8(h1 * 127.0f);
+                __syncthreads();
+                if (stop_s) {
+                    failed = true;
+                    break;
+                }
+            }
+            // ---- projection of the new layer-1 output
+            const float* h1 = kLong ? h_s[0] : h_s[(alt ^ 1) * 2 + 1];
+            float a = 0.0f;
+#pragma unroll
+            for (int j = 0; j < KP; ++j) {
+                const float2 v = *(const float2*)&h1[2 * lane + 128 * j];
+                a = __builtin_fmaf(lo16(wpj[j]), v.x, a);
+                a = __builtin_fmaf(hi16(wpj[j]), v.y, a);
+            }
+            a = wave_sum(a) + bpj;
+            if (lane == 0) out_s[1][wave] = a;
+            publish_out(pw, 1, tag);
+            if constexpr (kLong) {
+                // layer 1's recurrent sums of this candidate state, for the update after it is committed
+                uint32_t x[KD];
+#pragma unroll
+                for (int j = 0; j < KD; ++j) x[j] = 4 * lane + 256 * j < H ? q_s[1][lane + 64 * j] : 0u;
+                int d[4] = {0, 0, 0, 0};
+#pragma unroll
+                for (int g = 0; g < 4; ++g)
+#pragma unroll
+                    for (int j = 0; j < KD; ++j) d[g] = __builtin_amdgcn_sdot4((int)qw[1][g][j], (int)x[j], d[g], false);
+                const int s = row_isum4(d);
+                rs_next = half_row_isum(s + dpp_mov<0x128>(s));
+            }
+            pv = value(poll(pw + tid, 0xffffffffu, tag));
+            valid = true;
+        }
+        // ---- joint round: frames frame .. frame + kWin - 1 against this prediction
+#pragma unroll
+        for (int c = 0; c < kWin; ++c) {
+            const float e = g.frame + c < p.frames ? h2f(enc_s[(g.frame + c) & (k640Ring - 1)][tid]) : 0.0f;
+            x_s[c][tid] = __builtin_fmaxf(e + pv, 0.0f);
+        }
+        __syncthreads();
+        if (stop_s) {
+            failed = true;
+            break;
+        }
+        auto score_key = [&](float sum, float& score) -> u64 {
+            score = __builtin_fmaf(my_scale, sum, my_bias);
+            if (my_id < 0 || my_id >= T || score != score) return 0ull;
+            return ((u64)key_bits(score) << 32) | ((u64)(0xffffu - (uint32_t)my_id) << 16);
+        };
+        auto wpair = [&](int r, int j, float& w0, float& w1) {
+            if constexpr (kWide) {
+                w0 = __uint_as_float(wj[r][2 * j]);
+                w1 = __uint_as_float(wj[r][2 * j + 1]);
+            } else if constexpr (kInt8) {
+                w0 = (float)(int8_t)(wj[r][j / 2] >> (16 * (j & 1)));
+                w1 = (float)(int8_t)(wj[r][j / 2] >> (16 * (j & 1) + 8));
+            } else {
+                w0 = lo16(wj[r][j]);
+                w1 = hi16(wj[r][j]);
+            }
+        };
+        if (!extra) {
+            float acc[16];  // [frame][row]
+#pragma unroll
+            for (int i = 0; i < 16; ++i) acc[i] = 0.0f;
+#pragma unroll
+            for (int j = 0; j < KP; ++j)
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    const float2 x = *(const float2*)&x_s[4 * fh + c][2 * lane + 128 * j];
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        float w0, w1;
+                        wpair(r, j, w0, w1);
+                        acc[4 * c + r] = __builtin_fmaf(w0, x.x, acc[4 * c + r]);
+                        acc[4 * c + r] = __builtin_fmaf(w1, x.y, acc[4 * c + r]);
+                    }
+                }
+            float score;
+            u64 key = score_key(lanes_sum(acc, lane), score);
+            const int c = 4 * fh + ((lane >> 2) & 3);
+            if (lane < 16 && my_id >= T) dur_s[c][my_id - T] = score;  // workgroup 0 only
+            key = max_level(max_level(key, 1), 2);
+            if (lane < 16 && (lane & 3) == 0) key_s[c][wave & 3] = key;
+        } else if (my_id >= 0) {
+            float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int j = 0; j < KP; ++j)
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    const float2 x = *(const float2*)&x_s[4 * fh + c][2 * lane + 128 * j];
+                    float w0, w1;
+                    wpair(0, j, w0, w1);
+                    acc[c] = __builtin_fmaf(w0, x.x, acc[c]);
+                    acc[c] = __builtin_fmaf(w1, x.y, acc[c]);
+                }
+            float score;
+            const u64 key = score_key(lanes_sum(acc, lane), score);
+            if (lane < 4) key_s[4 * fh + lane][4] = key;
+        }
+        __syncthreads();
+        const uint32_t jtag = (rounds + 1) & 0x1fffu;
+        u64* jw = words(k640Joint) + (rounds & 1u) * (kWin * NB);  // [workgroup][window frame]
+        ++rounds;
+        if (wave == 0) {
+            // lanes 8 c .. 8 c + 7: the workgroup's key for window frame c
+            // (workgroup 0's with the first maximum of its duration scores)
+            const int c = lane >> 3;
+            u64 key = key_s[c][lane & 7];
+            key = max_level(max_level(max_level(key, 1), 2), 4);
+            if (blk == 0) {
+                float best = dur_s[c][0];
+                int d = 0;
+#pragma unroll
+                for (int i = 1; i < 8; ++i)
+                    if (i < D && dur_s[c][i] > best) {
+                        best = dur_s[c][i];
+                        d = i;
+                    }
+                key |= (u64)d << 13;
+            }
+            if ((lane & 7) == 0)
+                __hip_atomic_store(jw + blk * kWin + c, key | jtag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        if (wave < 8) {
+            // wave w: the keys of workgroups 8 w .. 8 w + 7
+            const u64 b = poll(jw + tid, 0x1fffu, jtag);
+            if (tid < kWin) win_dur[tid] = (int)((uint32_t)b >> 13) & 7;
+            const u64 m = max8(b);
+            if (lane < kWin) win_s[wave][lane] = m;
+        }
+        __syncthreads();
+        if (stop_s) {
+            failed = true;
+            break;
+        }
+        // identical in every wave
+        greedy_round(g, decisions(), blank, p.frames, p.max_symbols, [&](int token) {
+            if (blk == 0 && tid == 0 && count < p.capacity) p.tokens[count] = token;
+            ++count;
+            last = token;
+            emitted = true;
+            valid = false;
+            alt ^= 1;  // the candidate state becomes the committed one
+            c_cur[0] = c_new[0];
+            c_cur[1] = c_new[1];
+            rs = rs_next;
+            c0c = c0n;
+        });
+    }
+    if (blk == 0) {
+        ((float*)p.ws)[k640Out + tid] = pv;
+        if (tid == 0) {
+            p.result[0] = count;
+            p.result[1] = g.frame;
+            p.result[2] = failed ? -2 : 0;
+            p.result[3] = g.steps;
+        }
+    }
+}
+
 __global__ void decode_clear_kernel(uint32_t* ws, int words) {
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < words; i += gridDim.x * blockDim.x) ws[i] = 0u;
 }
@@ -800,6 +1482,16 @@ int launch_tdt_decode(const uint16_t* enc, int frames, int enc_stride, const uin
     a.max_symbols = max_symbols;
     a.capacity = capacity;
     decode_clear_kernel<<<16, 256, 0, s>>>(workspace, decode_workspace_words(hidden));
+    if (hidden == k640H && outputs <= k640Outputs && cu_count() >= k640Blocks) {
+        if (table) {
+            if (joint_int8) tdt_decode_640_kernel<true, true><<<k640Blocks, k640Threads, 0, s>>>(a);
+            else tdt_decode_640_kernel<false, true><<<k640Blocks, k640Threads, 0, s>>>(a);
+        } else {
+            if (joint_int8) tdt_decode_640_kernel<true, false><<<k640Blocks, k640Threads, 0, s>>>(a);
+            else tdt_decode_640_kernel<false, false><<<k640Blocks, k640Threads, 0, s>>>(a);
+        }
+        return 0;
+    }
     switch (hidden >> 7) {
 #define PK_DEC_CASE(KP)                                                                          \
     case KP:                                                                                     \
