@@ -15,9 +15,7 @@
 //           U4 probabilities x S4 values on the same instruction.
 //   tc:     fp16 scores on v_mfma_f32_16x16x32_f16; e4m3 probabilities x
 //           e4m3 values on v_mfma_scale_f32_16x16x128_f8f6f4.
-// Boundary tiles run the per-query FP32 path: one 32-lane half wave per
-// query, with the score, maximum and denominator reductions in the order of
-// the reference's 32-lane warps.
+// Boundary tiles run the fp32 tile kernel of pk_attention_tile.hpp.
 //
 // The MFMA reduction dimension may be permuted freely as long as both
 // operands use the same permutation (integer sums are exact).  The key and
@@ -26,6 +24,7 @@
 // kernel directly into the matching operand order.
 #include <float.h>
 
+#include "pk_attention_tile.hpp"
 #include "pk_common.hpp"
 #include "pk_kernels.hpp"
 
@@ -35,7 +34,6 @@ namespace {
 constexpr int kModel = 1024, kHead = 128, kHeads = 8;
 constexpr int kMaxAtt = 257, kPosRows = 272;
 constexpr float kScoreScale = 0.08838834764831845f;  // 1/sqrt(128)
-constexpr float kValueScale = 8.0f / 448.0f;         // FP8 V holds v * 56
 
 __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -112,17 +110,6 @@ __device__ __forceinline__ uint32_t pack_i8x4_biased(float a, float b, float c, 
     return ab | cd;
 }
 
-
-// Byte `b` of w as OCP e4m3 -> float (v_cvt_f32_fp8, exact); b folds to a
-// constant in unrolled loops.
-__device__ __forceinline__ float fp8_byte(uint32_t w, int b) {
-    switch (b) {
-        case 0: return __builtin_amdgcn_cvt_f32_fp8((int)w, 0);
-        case 1: return __builtin_amdgcn_cvt_f32_fp8((int)w, 1);
-        case 2: return __builtin_amdgcn_cvt_f32_fp8((int)w, 2);
-        default: return __builtin_amdgcn_cvt_f32_fp8((int)w, 3);
-    }
-}
 
 // e4m3 of two finite values (saturating), without the NaN handling of e4m3x2.
 __device__ __forceinline__ uint32_t e4m3x2_finite(float a, float b) {
@@ -316,120 +303,6 @@ struct TcShared {
     uint8_t prob[16][400];  // e4m3 probabilities for keys 0..383 (zero past the window)
     uint16_t out[16][128];
 };
-
-// Context store (encoder.cu:1463-1474) of two adjacent features: fp16 round,
-// packed form e4m3(x * 28).
-template <bool kPacked>
-__device__ __forceinline__ void store2(void* output, size_t index, float c0, float c1) {
-    if constexpr (kPacked)
-        *(uint16_t*)((uint8_t*)output + index) = (uint16_t)e4m3x2(round_f16(c0) * 28.0f, round_f16(c1) * 28.0f);
-    else
-        *(uint32_t*)((uint16_t*)output + index) = (uint32_t)f2h(c0) | ((uint32_t)f2h(c1) << 16);
-}
-
-// encoder.cu:1548-1684: the per-query FP32 path of boundary tiles, one wave
-// per query.  The arithmetic is the reference's, in its 32-lane warp order:
-// a slot's score is 16 partial sums (lane h of 16 accumulates dimensions
-// 2h + 32q, q = 0..3, interleaving content and position FMAs) reduced by a
-// shuffle tree; the denominator is 32 partial sums (partial l adds slots l,
-// l + 32, ... in order) reduced by a shuffle tree; each output feature's
-// context is one FMA chain over the keys in order.  Which lane runs which of
-// these chains is free, so a wave evaluates four slots per step, keeps eight
-// steps of loads in flight, and owns two features per lane.
-template <bool kPacked>
-__device__ void attention_query(float* scores, const uint16_t* __restrict__ query, const uint16_t* __restrict__ key,
-                                const uint8_t* __restrict__ value_fp8, const uint16_t* __restrict__ position,
-                                const uint16_t* __restrict__ bias_u, const uint16_t* __restrict__ bias_v, void* output, int qr,
-                                int head, int rows, int padded_rows, int valid_rows, int left, int right, int value_stride) {
-    const int lane = threadIdx.x & 63;
-    const size_t oidx = (size_t)qr * kModel + head * kHead + 2 * lane;
-    if (qr >= rows || qr >= valid_rows) {
-        if (qr < padded_rows) store2<kPacked>(output, oidx, 0.0f, 0.0f);
-        return;
-    }
-    const int first = max(0, qr - left), last = min(valid_rows - 1, qr + right);
-    const int count = last - first + 1;
-    const int grp = lane >> 4, hl = lane & 15;
-    float2 su[4], sv[4];
-#pragma unroll
-    for (int quarter = 0; quarter < 4; ++quarter) {
-        const int d = head * kHead + 2 * hl + 32 * quarter;
-        const uint32_t q = *(const uint32_t*)(query + (size_t)qr * kModel + d);
-        const uint32_t u = *(const uint32_t*)(bias_u + d);
-        const uint32_t v = *(const uint32_t*)(bias_v + d);
-        const float q0 = h2f((uint16_t)q), q1 = h2f((uint16_t)(q >> 16));
-        su[quarter] = make_float2(q0 + h2f((uint16_t)u), q1 + h2f((uint16_t)(u >> 16)));
-        sv[quarter] = make_float2(q0 + h2f((uint16_t)v), q1 + h2f((uint16_t)(v >> 16)));
-    }
-    constexpr int kU = 8;
-    for (int sp0 = 0; sp0 < count; sp0 += 4 * kU) {
-        uint32_t kw[kU][4], pw[kU][4];
-#pragma unroll
-        for (int u = 0; u < kU; ++u) {
-            const int key_row = first + min(sp0 + 4 * u + grp, count - 1);
-            const int prow = left - qr + key_row;
-#pragma unroll
-            for (int quarter = 0; quarter < 4; ++quarter) {
-                const int d = 2 * hl + 32 * quarter;
-                kw[u][quarter] = *(const uint32_t*)(key + (size_t)key_row * kModel + head * kHead + d);
-                pw[u][quarter] = *(const uint32_t*)(position + ((size_t)head * kPosRows + prow) * kHead + d);
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < kU; ++u) {
-            const int slot = sp0 + 4 * u + grp;
-            float s = 0.0f;
-#pragma unroll
-            for (int quarter = 0; quarter < 4; ++quarter) {
-                const uint32_t k = kw[u][quarter], p = pw[u][quarter];
-                s = __builtin_fmaf(su[quarter].x, h2f((uint16_t)k), s);
-                s = __builtin_fmaf(sv[quarter].x, h2f((uint16_t)p), s);
-                s = __builtin_fmaf(su[quarter].y, h2f((uint16_t)(k >> 16)), s);
-                s = __builtin_fmaf(sv[quarter].y, h2f((uint16_t)(p >> 16)), s);
-            }
-            s = sum_desc<16>(s);  // xor 8, 4, 2, 1
-            if (hl == 0 && slot < count) scores[slot] = s * kScoreScale;
-        }
-    }
-    wave_sync();
-    float mx = -FLT_MAX;
-    for (int slot = lane; slot < count; slot += 64) mx = __builtin_fmaxf(mx, scores[slot]);
-    mx = wave_max(mx);
-    for (int slot = lane; slot < count; slot += 64) scores[slot] = softmax_exp(scores[slot] - mx);
-    wave_sync();
-    float den = 0.0f;
-    if (lane < 32)
-        for (int slot = lane; slot < count; slot += 32) den += scores[slot];
-    den = sum_desc<32>(den);  // xor 16, ..., 1 over lanes 0..31
-    den = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(den)));
-    wave_sync();
-    for (int slot = lane; slot < count; slot += 64) scores[slot] = scores[slot] / den;
-    wave_sync();
-    float c0 = 0.0f, c1 = 0.0f;
-    const int feature = head * kHead + 2 * lane;
-    constexpr int kC = 16;  // chunks of four keys in flight per batch
-    for (int chunk0 = first & ~3; chunk0 <= last; chunk0 += 4 * kC) {
-        uint32_t words[kC][2];
-#pragma unroll
-        for (int b = 0; b < kC; ++b) {
-            const int chunk = min(chunk0 + 4 * b, last & ~3);
-            words[b][0] = *(const uint32_t*)(value_fp8 + (size_t)feature * value_stride + chunk);
-            words[b][1] = *(const uint32_t*)(value_fp8 + (size_t)(feature + 1) * value_stride + chunk);
-        }
-#pragma unroll
-        for (int b = 0; b < kC; ++b) {
-#pragma unroll
-            for (int item = 0; item < 4; ++item) {
-                const int kr = chunk0 + 4 * b + item;
-                if (kr < first || kr > last) continue;
-                const float weight = scores[kr - first];
-                c0 = __builtin_fmaf(weight, fp8_byte(words[b][0], item) * kValueScale, c0);
-                c1 = __builtin_fmaf(weight, fp8_byte(words[b][1], item) * kValueScale, c1);
-            }
-        }
-    }
-    store2<kPacked>(output, oidx, c0, c1);
-}
 
 // Softmax of query lq over its 257 slots from the combined logits held by a
 // half wave (lane ln has slots ln + 32 part).  Returns e = exp(l - max) in
@@ -804,22 +677,6 @@ __device__ void attention_tc_tile(TcShared& sh, const uint16_t* __restrict__ que
     }
 }
 
-// The boundary queries: tiles [0, ib) and [ie, tiles), four queries (one
-// per wave) of one head per workgroup, small LDS.
-template <bool kPacked>
-__global__ __launch_bounds__(256) void boundary_attention_kernel(
-    const uint16_t* __restrict__ query, const uint16_t* __restrict__ key, const uint8_t* __restrict__ value_fp8,
-    const uint16_t* __restrict__ position, const uint16_t* __restrict__ bias_u, const uint16_t* __restrict__ bias_v,
-    void* __restrict__ output, int rows, int padded_rows, int valid_rows, int left, int right, int value_stride, int ib, int ie) {
-    __shared__ QueryShared sh;
-    const int L = (int)blockIdx.x;
-    const int head = L & 7, grp = L >> 3, t = grp >> 2;
-    const int tile = t < ib ? t : ie + (t - ib);
-    attention_query<kPacked>(sh.scores[threadIdx.x >> 6], query, key, value_fp8, position, bias_u, bias_v, output,
-                             16 * tile + 4 * (grp & 3) + (int)(threadIdx.x >> 6), head, rows, padded_rows, valid_rows, left, right,
-                             value_stride);
-}
-
 // The interior tiles [ib, ie): packed -> `chunks` runs of consecutive tiles
 // per head, one workgroup each; tc -> one workgroup per tile and head.
 // Workgroup L runs on XCD L % 8; the work is split into eight contiguous
@@ -889,7 +746,7 @@ int launch_local_attention(bool packed, const uint16_t* query, const uint16_t* k
     const int hi = min(valid_rows - 16 - right, rows - 16);  // largest admissible qb
     const int ie = hi >= 16 * ib ? min(hi / 16 + 1, tiles) : ib;
     const int n = ie - ib;
-    const int boundary_wgs = 8 * 4 * (ib + (tiles - ie));
+    const int boundary_wgs = 8 * (ib + (tiles - ie));
     // Runs of consecutive tiles per head: two resident workgroups per CU
     // (the rings take 70 KB of LDS) for all eight heads.
     const int chunks = n > 0 ? max(1, min(n, 2 * cu_count() / 8)) : 1;
@@ -904,14 +761,11 @@ int launch_local_attention(bool packed, const uint16_t* query, const uint16_t* k
             interior_attention_kernel<false><<<interior_wgs, 256, 0, st>>>(query, key, value_fp8, position, bias_u, bias_v, output,
                                                                            value_stride, nullptr, nullptr, nullptr, nullptr, ib, ie, 1);
     };
+    const AttentionTileArgs edge{query, key, position, bias_u, bias_v, value_fp8, output, rows, padded_rows, valid_rows, left, right,
+                                 value_stride, ib, ie};
     auto boundary = [&](hipStream_t st) {
-        if (packed)
-            boundary_attention_kernel<true><<<boundary_wgs, 256, 0, st>>>(query, key, value_fp8, position, bias_u, bias_v, output, rows,
-                                                                          padded_rows, valid_rows, left, right, value_stride, ib, ie);
-        else
-            boundary_attention_kernel<false><<<boundary_wgs, 256, 0, st>>>(query, key, value_fp8, position, bias_u, bias_v, output,
-                                                                           rows, padded_rows, valid_rows, left, right, value_stride, ib,
-                                                                           ie);
+        if (packed) attention_tile_kernel<kTilePacked><<<boundary_wgs, kTileThreads, 0, st>>>(edge);
+        else attention_tile_kernel<kTileTc><<<boundary_wgs, kTileThreads, 0, st>>>(edge);
     };
     if (interior_wgs == 0 || boundary_wgs == 0) {
         if (interior_wgs) interior(s);
