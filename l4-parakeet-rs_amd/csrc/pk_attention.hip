@@ -275,26 +275,35 @@ __global__ __launch_bounds__(kValueThreads) void quantize_value_int4_kernel(cons
 
 // ---- attention -----------------------------------------------------------
 
-struct QueryShared {
-    float scores[4][264];  // one row per wave: scores, then exp, then weights
-};
 // Interior tiles of one head streamed through one workgroup: the keys and
-// S4 values of the current window live in rings indexed by key % 288 (the
-// 272-key window plus the 16 keys of the next tile), so each tile fetches only
-// its 16 new keys.
-constexpr int kRing = 288;
+// S4 values of the current window live in rings indexed by key % 272, so each
+// tile fetches only its 16 new keys, which take the slots of its 16 oldest
+// once the tile is done.  52 KiB, so that three workgroups share a CU (the
+// phases between barriers leave issue slots to the others: 45000 frames
+// 258 -> 228 us against two of 68 KiB): the quantized queries and then the U4
+// probabilities of row r lie in the position scores' rows, the outputs in the
+// content scores'.
+constexpr int kRing = 272;
 struct StreamShared {
-    uint8_t ring_k[kRing][72];  // INT4 key vectors (64 bytes, row padded)
+    uint8_t ring_k[kRing][64];   // INT4 key vectors, 16-byte chunks XOR-keyed by (slot / 4) % 4
     float ring_ks[kRing];
-    uint8_t ring_v[kHead][144];  // S4 V of the head's 128 features, ring key / 2
-    uint8_t qa_u[16][144];       // INT4 (q+u) as int8, MFMA operand order, rows padded
-    uint8_t qa_v[16][144];       // INT8 (q+v), reference score-vector byte order
-    uint16_t cs[16][kPosRows];
-    uint16_t ps[16][kPosRows];
-    uint8_t prob[16][336];  // U4 probabilities as bytes, prob_pos order
-    uint8_t out[16][128];
+    uint8_t ring_v[kHead][kRing / 2];  // S4 V of the head's 128 features, ring key / 2
+    union {
+        uint16_t cs[16][kPosRows];
+        uint8_t out[16][128];
+    };
+    union {
+        uint16_t ps[16][kPosRows];
+        uint8_t prob[16][2 * kPosRows];  // U4 probabilities as bytes, prob_pos order (336 of a row)
+        struct {
+            uint8_t qa_u[16][144];  // INT4 (q+u) as int8, MFMA operand order, rows padded
+            uint8_t qa_v[16][144];  // INT8 (q+v), reference score-vector byte order
+        };
+    };
     float qs_u[16], qs_v[16], pscale[16];
 };
+static_assert(3 * sizeof(StreamShared) <= 160 * 1024, "three workgroups per CU");
+__device__ __forceinline__ int ring_chunk(int slot, int chunk) { return ((chunk ^ (slot >> 2)) & 3) << 4; }
 struct TcShared {
     uint16_t qu[16][136];
     uint16_t qv[16][136];
@@ -363,7 +372,7 @@ __device__ void attention_packed_stream(StreamShared& sh, const uint16_t* __rest
         const int fk = 16 * t0 - 128;
         for (int i = tid; i < kPosRows * 4; i += 256) {
             const int key = fk + (i >> 2);
-            *(uint4*)&sh.ring_k[key % kRing][16 * (i & 3)] =
+            *(uint4*)&sh.ring_k[key % kRing][ring_chunk(key % kRing, i & 3)] =
                 *(const uint4*)(packed_key + ((size_t)key * kHeads + head) * 64 + 16 * (i & 3));
         }
         for (int i = tid; i < kPosRows; i += 256) sh.ring_ks[(fk + i) % kRing] = key_scales[(size_t)(fk + i) * kHeads + head];
@@ -379,8 +388,7 @@ __device__ void attention_packed_stream(StreamShared& sh, const uint16_t* __rest
         const int qb = 16 * t, first_key = qb - 128;
         const bool more = t + 1 < t1;
 
-        // Phase 1: clear the probability rows; quantize q+u and q+v.
-        for (int i = tid; i < 16 * 336 / 4; i += 256) ((uint32_t*)sh.prob)[i] = 0;
+        // Phase 1: quantize q+u and q+v.
         {
             // q+u and q+v as fp16 adds: for fp16 operands, rounding the fp32 sum
             // to fp16 is the same as one fp16 addition (24 >= 2*11 + 2 bits).
@@ -454,6 +462,7 @@ __device__ void attention_packed_stream(StreamShared& sh, const uint16_t* __rest
                 qsu[r] = sh.qs_u[4 * g + r];
                 qsv[r] = sh.qs_v[4 * g + r];
             }
+            __syncthreads();  // the scores overwrite the quantized queries
             const int ring0 = first_key % kRing;
 #pragma unroll
             for (int i = 0; i < 5; ++i) {
@@ -461,7 +470,8 @@ __device__ void attention_packed_stream(StreamShared& sh, const uint16_t* __rest
                 const int col = 16 * kt + l16;
                 int slot = ring0 + col;
                 slot = slot >= kRing ? slot - kRing : slot;
-                const uint2 k0 = *(const uint2*)&sh.ring_k[slot][8 * g], k1 = *(const uint2*)&sh.ring_k[slot][32 + 8 * g];
+                const uint2 k0 = *(const uint2*)&sh.ring_k[slot][ring_chunk(slot, g >> 1) + 8 * (g & 1)];
+                const uint2 k1 = *(const uint2*)&sh.ring_k[slot][ring_chunk(slot, 2 + (g >> 1)) + 8 * (g & 1)];
                 const float ks = sh.ring_ks[slot], pscl = psc[i];
                 // |sums| <= 7 * 128 * 128 (INT4 x widened INT4) and 127 * 127 * 128 (INT8), below 2^22
                 const v4i bias = v4i{kIntBias, kIntBias, kIntBias, kIntBias};
@@ -510,6 +520,13 @@ __device__ void attention_packed_stream(StreamShared& sh, const uint16_t* __rest
             }
             const float den = row_sum_tree16(even + odd);
             if (j == 0) sh.pscale[lq] = 1.0f / (15.0f * den);
+            // the row's position scores are in registers: its probabilities take
+            // their place (zero outside the window)
+            uint32_t* zrow = (uint32_t*)sh.prob[lq];
+#pragma unroll
+            for (int k = 0; k < 6; ++k)
+                if (j + 16 * k < 336 / 4) zrow[j + 16 * k] = 0u;
+            wave_sync();
             uint8_t* prow = &sh.prob[lq][prob_pos(lq + j)];  // slot j + 16k sits 16k further
 #pragma unroll
             for (int k = 0; k < 17; ++k)
@@ -554,10 +571,10 @@ __device__ void attention_packed_stream(StreamShared& sh, const uint16_t* __rest
         }
         __syncthreads();
         *(uint2*)(output + (size_t)(qb + qr16) * kModel + head * kHead + 8 * qj) = *(const uint2*)&sh.out[qr16][8 * qj];
-        // The 16 new keys go to ring slots of keys qb-144 .. qb-129, which this
-        // tile no longer reads; the next tile's first barrier publishes them.
+        // The 16 new keys go to the ring slots of keys qb-128 .. qb-113, which no
+        // tile reads any more; the next tile's first barrier publishes them.
         if (more) {
-            if (tid < 64) *(uint4*)&sh.ring_k[(nkey + (tid >> 2)) % kRing][16 * (tid & 3)] = nk;
+            if (tid < 64) *(uint4*)&sh.ring_k[(nkey + (tid >> 2)) % kRing][ring_chunk((nkey + (tid >> 2)) % kRing, tid & 3)] = nk;
             else if (tid < 80) sh.ring_ks[(nkey + tid - 64) % kRing] = nks;
             else if (tid >= 128) *(uint2*)&sh.ring_v[tid - 128][(nkey % kRing) / 2] = nv;
         }
@@ -683,7 +700,7 @@ __device__ void attention_tc_tile(TcShared& sh, const uint16_t* __restrict__ que
 // ranges of (tile or run, head) pairs so that each XCD's L2 holds the keys
 // and values of neighbouring tiles.
 template <bool kPacked>
-__global__ __launch_bounds__(256) void interior_attention_kernel(
+__global__ __launch_bounds__(256, kPacked ? 3 : 2) void interior_attention_kernel(
     const uint16_t* __restrict__ query, const uint16_t* __restrict__ key, const uint8_t* __restrict__ value_fp8,
     const uint16_t* __restrict__ position, const uint16_t* __restrict__ bias_u, const uint16_t* __restrict__ bias_v,
     void* __restrict__ output, int value_stride, const uint8_t* __restrict__ packed_key, const float* __restrict__ key_scales,
@@ -747,9 +764,9 @@ int launch_local_attention(bool packed, const uint16_t* query, const uint16_t* k
     const int ie = hi >= 16 * ib ? min(hi / 16 + 1, tiles) : ib;
     const int n = ie - ib;
     const int boundary_wgs = 8 * (ib + (tiles - ie));
-    // Runs of consecutive tiles per head: two resident workgroups per CU
-    // (the rings take 70 KB of LDS) for all eight heads.
-    const int chunks = n > 0 ? max(1, min(n, 2 * cu_count() / 8)) : 1;
+    // Runs of consecutive tiles per head: three resident workgroups per CU
+    // (52 KiB of LDS each) for all eight heads.
+    const int chunks = n > 0 ? max(1, min(n, 3 * cu_count() / 8)) : 1;
     const int interior_wgs = n > 0 ? 8 * (packed ? chunks : n) : 0;
 
     auto interior = [&](hipStream_t st) {
