@@ -199,13 +199,128 @@ __global__ __launch_bounds__(256) void pack_vectors_kernel(const uint16_t* __res
     }
 }
 
-// encoder.cu:561-634.  One 256-thread workgroup per feature row of the
-// feature-major V [1024 x rows], 8 consecutive keys per thread and pass: the
-// first pass takes the row's maximum, the second re-reads the row and
-// quantizes it.  Few registers, so all 1024 workgroups are resident at once.
-// Measured ≈ 49 µs at T = 45000 (2.4 TB/s of algorithmic bytes), the same as a
-// register-resident single pass with 1024-thread workgroups, deeper unrolling
-// or rotated start offsets.
+// encoder.cu:561-634, rows that one workgroup holds in registers: one read of
+// V, 8 kPer keys a thread.  HBM-bound once the arithmetic is short (2560
+// bytes a frame: 22 us at T = 45000 at the rate of a large copy): the maximum
+// is a packed integer one of the halves' magnitudes, and a value costs two
+// fmas on the packed half (its rounded quotient in the low bits of the float
+// 1.5 * 2^23 + q, and the distance from it), a subtraction and half a maximum;
+// rows with infinities or NaN, and groups of eight with a near-tie, take the
+// division.  T = 45000: 47 -> 26 us (two passes over the row, fifteen
+// operations a value).
+template <int kThreads, int kPer>
+__global__ __launch_bounds__(kThreads) void quantize_value_reg_kernel(const uint16_t* __restrict__ vt, uint8_t* __restrict__ out,
+                                                                     int rows, float inverse_scale, int edge_only, int valid_rows) {
+    const int f = blockIdx.x, tid = threadIdx.x;
+    const size_t elements = (size_t)rows * kModel;
+    const uint16_t* x = vt + (size_t)f * rows;
+    __shared__ uint32_t wave_s[kThreads / 64];
+    typedef uint16_t u16x2_t __attribute__((ext_vector_type(2)));
+    auto umax2 = [](uint32_t p, uint32_t q) {  // larger of each pair of 16-bit halves
+        return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2_t, p), __builtin_bit_cast(u16x2_t, q)));
+    };
+    uint4 d[kPer];
+    uint32_t m2 = 0;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+        const int r = 8 * (tid + kThreads * i);
+        d[i] = r < rows ? *(const uint4*)(x + r) : uint4{0, 0, 0, 0};
+    }
+#pragma unroll
+    for (int i = 0; i < kPer; ++i)
+        m2 = umax2(umax2(umax2(d[i].x & 0x7fff7fffu, d[i].y & 0x7fff7fffu), umax2(d[i].z & 0x7fff7fffu, d[i].w & 0x7fff7fffu)), m2);
+    int m1 = (int)max(m2 & 0xffffu, m2 >> 16);
+#pragma unroll
+    for (int off = 1; off <= 32; off <<= 1) {
+        if (off <= 8) {
+            m1 = max(m1, partner(m1, off));
+        } else {
+            int p, q;
+            pair_of(m1, off, p, q);
+            m1 = max(p, q);
+        }
+    }
+    if ((tid & 63) == 0) wave_s[tid >> 6] = (uint32_t)m1;
+    __syncthreads();
+    uint32_t bits = 0;
+#pragma unroll
+    for (int i = 0; i < kThreads / 64; ++i) bits = max(bits, wave_s[i]);
+    bits = __builtin_amdgcn_readfirstlane(bits);
+    const bool odd_row = bits >= 0x7c00u;  // an infinity or NaN in the row
+    float top = h2f((uint16_t)bits);
+    if (odd_row) {
+        // fmax ignores NaN: the largest magnitude that is a number
+        __syncthreads();
+        float m = 0.0f;
+#pragma unroll
+        for (int i = 0; i < kPer; ++i) {
+            const uint32_t w[4] = {d[i].x, d[i].y, d[i].z, d[i].w};
+#pragma unroll
+            for (int j = 0; j < 8; ++j) m = __builtin_fmaxf(m, __builtin_fabsf(h2f((uint16_t)(w[j / 2] >> (16 * (j & 1))))));
+        }
+        m = wave_max(m);
+        if ((tid & 63) == 0) wave_s[tid >> 6] = __float_as_uint(m);
+        __syncthreads();
+        top = 0.0f;
+#pragma unroll
+        for (int i = 0; i < kThreads / 64; ++i) top = __builtin_fmaxf(top, __uint_as_float(wave_s[i]));
+    }
+    const float scale = top > 0.0f ? top / 7.0f : 1.0f;
+    if (tid == 0) ((float*)(out + elements + elements / 2))[f] = scale;
+    const float inv = __builtin_amdgcn_rcpf(scale);
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+        const int r = 8 * (tid + kThreads * i);
+        if (r >= rows) break;
+        const uint32_t w[4] = {d[i].x, d[i].y, d[i].z, d[i].w};
+        uint32_t q[8];
+        float far = 0.0f;
+        const bool any8 = !edge_only || r < 272 || r + 7 >= valid_rows - 272;  // some pair stores FP8
+        if (!odd_row) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const float v = h2f((uint16_t)(w[j / 2] >> (16 * (j & 1))));
+                const float n = __builtin_fmaf(v, inv, kFloatBias);
+                q[j] = __float_as_uint(n);
+                far = __builtin_fmaxf(far, __builtin_fabsf(__builtin_fmaf(v, inv, kFloatBias - n)));
+            }
+        }
+        if (odd_row || __builtin_amdgcn_ballot_w64(far > 0.49995f) != 0) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                // clamp(rn(v / s), -7, 7); a NaN input quantizes to 0
+                const float v = h2f((uint16_t)(w[j / 2] >> (16 * (j & 1))));
+                q[j] = v != v ? 0u : (uint32_t)(int)__builtin_fminf(__builtin_fmaxf(__builtin_rintf(v / scale), -7.0f), 7.0f);
+            }
+        }
+        // nibbles of keys 2 p, 2 p + 1 to byte p
+        uint32_t b[4];
+#pragma unroll
+        for (int p = 0; p < 4; ++p) b[p] = (q[2 * p] & 15u) | (q[2 * p + 1] << 4);
+        const uint32_t lo = __builtin_amdgcn_perm(b[1], b[0], 0x0c0c0400u), hi = __builtin_amdgcn_perm(b[3], b[2], 0x04000c0cu);
+        *(uint32_t*)(out + elements + ((size_t)f * rows + r) / 2) = lo | hi;
+        if (!any8) continue;
+        uint32_t fp8[4];
+        bool all = true;
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+            fp8[p] = e4m3x2(h2f((uint16_t)w[p]) * inverse_scale, h2f((uint16_t)(w[p] >> 16)) * inverse_scale);
+            all = all && (!edge_only || r + 2 * p < 272 || r + 2 * p + 1 >= valid_rows - 272);
+        }
+        uint8_t* o = out + (size_t)f * rows + r;
+        if (all) {
+            *(uint2*)o = uint2{fp8[0] | (fp8[1] << 16), fp8[2] | (fp8[3] << 16)};
+        } else {
+#pragma unroll
+            for (int p = 0; p < 4; ++p)
+                if (r + 2 * p < 272 || r + 2 * p + 1 >= valid_rows - 272) *(uint16_t*)(o + 2 * p) = (uint16_t)fp8[p];
+        }
+    }
+}
+
+// The same for longer rows, in two passes over the row: 8 consecutive keys per
+// thread and pass, the first takes the row's maximum, the second re-reads the
+// row and quantizes it.
 constexpr int kValueThreads = 256;
 __global__ __launch_bounds__(kValueThreads) void quantize_value_int4_kernel(const uint16_t* __restrict__ vt, uint8_t* __restrict__ out,
                                                                            int rows, float inverse_scale, int edge_only,
@@ -748,7 +863,20 @@ int launch_pack_vectors(bool int4, const uint16_t* in, uint8_t* out, float* scal
 
 int launch_quantize_value_int4(const uint16_t* vt, uint8_t* out, int rows, float inverse_scale, bool edge_only, int valid_rows,
                                hipStream_t s) {
-    quantize_value_int4_kernel<<<kModel, kValueThreads, 0, s>>>(vt, out, rows, inverse_scale, edge_only ? 1 : 0, valid_rows);
+    // by what a thread holds: 2, 4 or 8 chunks of 8 keys (256 threads: 16384
+    // rows), then 1024 threads (65536 rows, two workgroups a CU)
+    const int chunks = (rows + 7) / 8;
+#define PK_VALUE_REG(threads, per) \
+    quantize_value_reg_kernel<threads, per><<<kModel, threads, 0, s>>>(vt, out, rows, inverse_scale, edge_only ? 1 : 0, valid_rows)
+    if (chunks <= 256) PK_VALUE_REG(256, 1);
+    else if (chunks <= 256 * 4) PK_VALUE_REG(256, 4);
+    else if (chunks <= 256 * 8) PK_VALUE_REG(256, 8);
+    else if (chunks <= 1024 * 4) PK_VALUE_REG(1024, 4);
+    else if (chunks <= 1024 * 6) PK_VALUE_REG(1024, 6);
+    else if (chunks <= 1024 * 8) PK_VALUE_REG(1024, 8);
+    else
+        quantize_value_int4_kernel<<<kModel, kValueThreads, 0, s>>>(vt, out, rows, inverse_scale, edge_only ? 1 : 0, valid_rows);
+#undef PK_VALUE_REG
     return 0;
 }
 

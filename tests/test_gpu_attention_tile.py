@@ -50,3 +50,27 @@ def test_tile_non_finite_values(pk, orc, bad):  # noqa: F811
     assert not np.isfinite(got[~clean]).any()
     assert np.isfinite(got[clean]).all()
     assert np.abs(got - ref)[clean].max() <= TOL * np.sqrt((ref ** 2).mean())
+
+
+@pytest.mark.parametrize("rows,edge", [(16, True), (2048, False), (2064, True), (8208, True), (16400, False), (32784, True), (49168, False),
+                                       (65536, True), (65552, True)])
+def test_value_quantizer_row_sizes(pk, orc, rows, edge):  # noqa: F811
+    """Rows at and one step past what a workgroup of each size holds, with
+    near-ties (multiples of half a step), infinities and NaN: bit for bit."""
+    gen = torch.Generator().manual_seed(rows)
+    vt = torch.randn((1024, rows), generator=gen).half()
+    vt[1::5] = (torch.randint(-14, 15, vt[1::5].shape, generator=gen) * 0.5).half()  # v / s at half-integers
+    vt[1::5, 0] = 7.0
+    vt[7, rows // 2], vt[12, 3], vt[12, 4], vt[17], vt[22] = float("nan"), float("inf"), float("nan"), 0, 6e-8
+    vt = vt.numpy()
+    el = rows * 1024
+    out = torch.full((el + el // 2 + 4096,), 0xAB, dtype=torch.uint8, device="cuda")
+    if edge:
+        pk.call("pk_quantize_value_int4_register", dev(vt), out, el, 56.0, rows - 3)
+    else:
+        pk.call("pk_quantize_value_int4", dev(vt), out, el, 56.0)
+    ref = orc.quantize_value_int4(vt, 56.0, edge_only=edge, valid_rows=rows - 3 if edge else rows, fill=0xAB)
+    # a NaN quantizes to 0 (the oracle's conversion of NaN to int is not defined)
+    for f, r in np.argwhere(np.isnan(vt)):
+        ref[el + (f * rows + r) // 2] &= 0x0F if r & 1 else 0xF0
+    np.testing.assert_array_equal(host(out), ref)
