@@ -92,7 +92,30 @@ static int launch_ring(const GemmArgs& a, hipStream_t s) {
     return 0;
 }
 
-// The ring kernel with two waves per SIMD (FP8 / INT8, 64- or 128-row tiles;
+// The same two K-steps at a time.
+template <int F, int E, int kAI>
+static int launch_ring_pair(const GemmArgs& a, hipStream_t s) {
+    using L = g3::LP<F, kAI>;
+    static std::once_flag once;
+    static hipError_t attr = hipSuccess;
+    std::call_once(once, [] {
+        attr = hipFuncSetAttribute((const void*)g3::gemm3_ring_pair_kernel<F, E, kAI>, hipFuncAttributeMaxDynamicSharedMemorySize, L::kBytes);
+    });
+    if (attr != hipSuccess) {
+        set_error("hipFuncSetAttribute(LDS %d bytes) failed: %s", L::kBytes, hipGetErrorString(attr));
+        return -3;
+    }
+    const int tiles = ((a.m + L::kBM - 1) / L::kBM) * ((a.n + g3::kBN - 1) / g3::kBN);
+    hipLaunchKernelGGL((g3::gemm3_ring_pair_kernel<F, E, kAI>), dim3(tiles), dim3(g3::kThreads), L::kBytes, s, a);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) {
+        set_error("gemm launch (fmt %d, epi %d) failed: %s", F, E, hipGetErrorString(e));
+        return -3;
+    }
+    return 0;
+}
+
+// The ring kernel with two waves per SIMD (FP8 / INT8, 128-row tiles, and 64-row ones of an odd number of K-steps;
 // measured slower for INT4-g128 x fp16 on 96-row tiles, split 2 : 1, 19.6 ->
 // 22.6 us, and for INT4-g128 x INT8 on 128-row tiles against its two 64-row
 // ring workgroups per CU, 13.4 -> 13.9 us).
@@ -256,6 +279,10 @@ static int tile_plan(int fmt, int epi, int m, int n, int* cols, int* stages) {
             return r;
         }
     }
+    if (fmt == FMT_FP8 && epi == EPI_GLU && ring_rows(fmt, m, n)) {
+        *stages = ring_stages(fmt, ring_rows(fmt, m, n) / 32);
+        return ring_rows(fmt, m, n);
+    }
     if (fmt == FMT_Q4K || (fmt == FMT_FP8 && epi == EPI_GLU)) {
         *cols = kBlockN;
         return kBlockM;
@@ -291,6 +318,11 @@ static int launch_fmt(const GemmArgs& a, hipStream_t s) {
                 }
                 if constexpr (F == FMT_FP8 || F == FMT_I8) {
                     // two waves per SIMD (C1: 11.1 -> 10.0 us; FP8 750 x 1024 -> 4096: 10.9 -> 9.5)
+                    // two K-steps per barrier on 32 and 64 rows (FP8: 96 x 1024 x 4096 16.3 ->
+                    // 11.7 us, 96 x 4096 x 1024 7.0 -> 5.8, 496 x 3072 x 1024 8.9 -> 8.6); on 128
+                    // rows the two waves per SIMD hide more (752 x 4096 x 1024: 10.0 against 10.9)
+                    if (a.k % 256 == 0 && rows == 32) return launch_ring_pair<F, E, 1>(a, s);
+                    if (a.k % 256 == 0 && rows == 64) return launch_ring_pair<F, E, 2>(a, s);
                     if (rows == 64) return launch_ring8<F, E, 2>(a, s);
                     if (rows == 128) return launch_ring8<F, E, 4>(a, s);
                 }
@@ -348,6 +380,13 @@ static int by_epi(int epi, const GemmArgs& a, hipStream_t s) {
                 set_error("GLU needs n %% 256 == 0 weight rows, ldo == n/2 and weight scales");
                 return -1;
             }
+            // Small grids: one tile of 128 weight rows per workgroup.  752 frames (K =
+            // 1024) 16.4 -> 6.1 us on 64 rows, 96 frames 14.1 -> 4.7 on 32; 256 x 256 tiles
+            // leave all but 24 CUs idle.
+            const int rows = ring_rows(FMT_FP8, a.m, a.n);
+            if (rows == 32) return a.k % 256 == 0 ? launch_ring_pair<F, EPI_GLU, 1>(a, s) : launch_ring<F, EPI_GLU, 1>(a, s);
+            if (rows == 64) return a.k % 256 == 0 ? launch_ring_pair<F, EPI_GLU, 2>(a, s) : launch_ring8<F, EPI_GLU, 2>(a, s);
+            if (rows == 128) return launch_ring8<F, EPI_GLU, 4>(a, s);
             return launch_one<F, EPI_GLU>(a, s);
         }
         break;

@@ -688,13 +688,14 @@ __device__ __forceinline__ int glu_row(int n0, int L, int n) {
 
 // GLU epilogue: out[row, c + j] = fp16(fp16(v_j) / (1 + exp(-fp16(g_j)))),
 // rows >= valid_rows written as zero (encoder.cu:936-947).
-__device__ __forceinline__ void epilogue_glu(const GemmArgs& p, v4f (&accf)[8][4], int m0, int n0, int wm, int wn, int lane) {
+template <int kAI = 8>
+__device__ __forceinline__ void epilogue_glu(const GemmArgs& p, v4f (&accf)[kAI][4], int m0, int n0, int wm, int wn, int lane) {
     const int g = lane >> 4, l16 = lane & 15;
     const int half = p.n >> 1;
     const int oc = (n0 >> 1) + ((wn * 4 + g) << 3);  // first of the lane's 8 output columns
     const bool col_live = oc < half;
     const int cc = min(oc, half - 8);
-    float wv[8], wg[8], rsv[8];
+    float wv[8], wg[8], rsv[kAI];
 #pragma unroll
     for (int j = 0; j < 8; j += 4) {
         const float4 a = *(const float4*)(p.w_scales + cc + j);
@@ -703,14 +704,14 @@ __device__ __forceinline__ void epilogue_glu(const GemmArgs& p, v4f (&accf)[8][4
         wg[j] = b.x; wg[j + 1] = b.y; wg[j + 2] = b.z; wg[j + 3] = b.w;
     }
 #pragma unroll
-    for (int ai = 0; ai < 8; ++ai) {
-        const int row = min(m0 + wm * 128 + ai * 16 + l16, p.m - 1);
+    for (int ai = 0; ai < kAI; ++ai) {
+        const int row = min(m0 + wm * 16 * kAI + ai * 16 + l16, p.m - 1);
         rsv[ai] = p.row_scales ? p.row_scales[row] : p.in_scale;
     }
     __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
 #pragma unroll
-    for (int ai = 0; ai < 8; ++ai) {
-        const int grow = m0 + wm * 128 + ai * 16 + l16;
+    for (int ai = 0; ai < kAI; ++ai) {
+        const int grow = m0 + wm * 16 * kAI + ai * 16 + l16;
         const float rs = rsv[ai];
         uint32_t h[4];
 #pragma unroll
