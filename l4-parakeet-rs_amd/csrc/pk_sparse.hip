@@ -11,8 +11,12 @@
 // the reference's 2:4 rows are consumed as they are stored.
 //
 // Workgroup tile 256 x 256 (8 waves, 128 x 64 each), persistent over tiles,
-// direct-to-LDS loads, double-buffered stages of 16 KiB compressed data +
-// 4 KiB metadata + 32 KiB weights.  Weight row n(j, bj) = 4j + bj feeds MFMA
+// direct-to-LDS loads into a ring of three stages of 16 KiB compressed data +
+// 4 KiB metadata + 32 KiB weights, so that a stage has two steps to land.  A
+// step takes 1.35 us whatever the grid (1024 cycles of MFMA a wave, two waves
+// a SIMD); two stages and a residual load behind every store: 45000 frames
+// 178 -> 156 us, 20000 108 -> 94, 7500 55 -> 47.  128-row tiles measured 43 us a
+// round against 45 and are not used.  Weight row n(j, bj) = 4j + bj feeds MFMA
 // column j of block bj, so each lane's accumulators for one 16-row block are
 // 4 rows x 4 contiguous output columns.
 #include "pk_kernels.hpp"
@@ -23,6 +27,7 @@ constexpr int kSpData = 256 * 64;     // compressed activation bytes per stage
 constexpr int kSpMeta = 256 * 16;     // metadata bytes per stage
 constexpr int kSpW = 256 * 128;       // weight bytes per stage
 constexpr int kSpStage = kSpData + kSpMeta + kSpW;
+constexpr int kSpStages = 3;          // 156 KiB
 
 // XOR key of a 64-byte compressed row's 16-byte chunks: 8 (16) consecutive
 // rows reading one chunk column touch distinct banks of 128 (256) bytes.
@@ -55,7 +60,7 @@ struct SparseArgs {
 
 __global__ __launch_bounds__(kThreads, 1) void sparse24_contract_kernel(SparseArgs p) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave >> 2, wn = wave & 3;
     const int g = lane >> 4, l16 = lane & 15;
     const int tiles_n = (p.n + kBlockN - 1) / kBlockN;
@@ -72,12 +77,15 @@ __global__ __launch_bounds__(kThreads, 1) void sparse24_contract_kernel(SparseAr
     // 128-byte rows swizzled by spw_key).
     uint32_t d_off[2], m_off = 0, w_off[4];
     const int gw = group_width(tiles_n);
-    auto set_tile = [&](int t, int& m0, int& n0) {
+    auto tile_origin = [&](int t, int& m0, int& n0) {
         const int ng = t / (tiles_m * gw);
         const int r = t - ng * tiles_m * gw;
         const int tm = r / gw;
         m0 = tm * kBlockM;
         n0 = (ng * gw + (r - tm * gw)) * kBlockN;
+    };
+    auto set_tile = [&](int t, int& m0, int& n0) {
+        tile_origin(t, m0, n0);
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
             const int o = (wave * 2 + i) * 1024 + lane * 16;
@@ -104,11 +112,22 @@ __global__ __launch_bounds__(kThreads, 1) void sparse24_contract_kernel(SparseAr
         for (int i = 0; i < 4; ++i) dma16(p.w + w_off[i] + (size_t)step * 128, base + kSpData + kSpMeta + (wave * 4 + i) * 1024);
     };
 
-    int t = tile_slot(G);
-    if (t >= ntiles) return;
-    int m0, n0;
+    // The load stream runs kSpStages - 1 steps ahead of the MFMAs, across tiles.
+    int lt = tile_slot(G), lstep = 0, lbuf = 0;
+    if (lt >= ntiles) return;
+    int t = lt, m0, n0, lm0, ln0;
     set_tile(t, m0, n0);
-    issue(0, 0);
+    auto issue_next = [&]() {
+        if (lt >= ntiles) return;
+        issue(lstep, lbuf);
+        lbuf = lbuf + 1 == kSpStages ? 0 : lbuf + 1;
+        if (++lstep == steps) {
+            lstep = 0;
+            lt += G;
+            if (lt < ntiles) set_tile(lt, lm0, ln0);
+        }
+    };
+    for (int i = 0; i < kSpStages - 1; ++i) issue_next();
     int buf = 0;
     v4f acc[8][4];
 
@@ -121,14 +140,13 @@ __global__ __launch_bounds__(kThreads, 1) void sparse24_contract_kernel(SparseAr
             for (int j = 0; j < 4; ++j) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
 
         for (int step = 0; step < steps; ++step) {
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            // this wave's loads of the stage have landed (those of the next one,
+            // 7 or 6, may be in flight; the last stages wait for everything)
+            if (t_next >= ntiles && step + 2 > steps) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            else if (wave < 4) asm volatile("s_waitcnt vmcnt(7)" ::: "memory");
+            else asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
             __syncthreads();
-            if (step + 1 < steps) {
-                issue(step + 1, buf ^ 1);
-            } else if (t_next < ntiles) {
-                set_tile(t_next, m0, n0);
-                issue(0, buf ^ 1);
-            }
+            issue_next();
             const uint8_t* Ds = lds + buf * kSpStage;
             const uint8_t* Ms = Ds + kSpData;
             const uint8_t* Ws = Ms + kSpMeta;
@@ -149,7 +167,7 @@ __global__ __launch_bounds__(kThreads, 1) void sparse24_contract_kernel(SparseAr
 #pragma unroll
                 for (int bj = 0; bj < 4; ++bj) acc[ai][bj] = __builtin_amdgcn_smfmac_f32_16x16x128_fp8_fp8(dv, wf[bj], acc[ai][bj], idx, 0, 0);
             }
-            buf ^= 1;
+            buf = buf + 1 == kSpStages ? 0 : buf + 1;
         }
 
         // Epilogue: lane holds rows 4g + r of each 16-row block and columns
@@ -158,24 +176,39 @@ __global__ __launch_bounds__(kThreads, 1) void sparse24_contract_kernel(SparseAr
         const bool col_live = gcol < p.n;
         const float4 ws = *(const float4*)(p.w_scales + min(gcol, p.n - 4));
         const float wsv[4] = {ws.x, ws.y, ws.z, ws.w};
+        // Residuals are loaded four row blocks at a time before those blocks' stores:
+        // the compiler keeps a load of `out` behind an earlier store to it, and 32
+        // round trips to memory followed one another.
 #pragma unroll
-        for (int ai = 0; ai < 8; ++ai) {
+        for (int a0 = 0; a0 < 8; a0 += 4) {
+            uint2 res[4][4];
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int grow = cur_m0 + wm * 128 + ai * 16 + 4 * g + r;
-                if (grow >= p.m || !col_live) continue;
-                uint16_t* o = p.out + (size_t)grow * p.n + gcol;
-                const uint2 res = *(const uint2*)o;
-                const float r0 = h2f((uint16_t)(res.x & 0xffff)), r1 = h2f((uint16_t)(res.x >> 16));
-                const float r2 = h2f((uint16_t)(res.y & 0xffff)), r3 = h2f((uint16_t)(res.y >> 16));
-                const float v0 = acc[ai][0][r] * p.in_scale * wsv[0], v1 = acc[ai][1][r] * p.in_scale * wsv[1];
-                const float v2 = acc[ai][2][r] * p.in_scale * wsv[2], v3 = acc[ai][3][r] * p.in_scale * wsv[3];
-                *(uint2*)o = uint2{(uint32_t)f2h(__builtin_fmaf(0.5f, v0, r0)) | ((uint32_t)f2h(__builtin_fmaf(0.5f, v1, r1)) << 16),
-                                   (uint32_t)f2h(__builtin_fmaf(0.5f, v2, r2)) | ((uint32_t)f2h(__builtin_fmaf(0.5f, v3, r3)) << 16)};
-            }
+            for (int ai = 0; ai < 4; ++ai)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int grow = min(cur_m0 + wm * 128 + (a0 + ai) * 16 + 4 * g + r, p.m - 1);
+                    res[ai][r] = *(const uint2*)(p.out + (size_t)grow * p.n + min(gcol, p.n - 4));
+                }
+#pragma unroll
+            for (int ai = 0; ai < 4; ++ai)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int grow = cur_m0 + wm * 128 + (a0 + ai) * 16 + 4 * g + r;
+                    if (grow >= p.m || !col_live) continue;
+                    const uint2 x = res[ai][r];
+                    const float r0 = h2f((uint16_t)(x.x & 0xffff)), r1 = h2f((uint16_t)(x.x >> 16));
+                    const float r2 = h2f((uint16_t)(x.y & 0xffff)), r3 = h2f((uint16_t)(x.y >> 16));
+                    const v4f(&c)[4] = acc[a0 + ai];
+                    const float v0 = c[0][r] * p.in_scale * wsv[0], v1 = c[1][r] * p.in_scale * wsv[1];
+                    const float v2 = c[2][r] * p.in_scale * wsv[2], v3 = c[3][r] * p.in_scale * wsv[3];
+                    *(uint2*)(p.out + (size_t)grow * p.n + gcol) =
+                        uint2{(uint32_t)f2h(__builtin_fmaf(0.5f, v0, r0)) | ((uint32_t)f2h(__builtin_fmaf(0.5f, v1, r1)) << 16),
+                              (uint32_t)f2h(__builtin_fmaf(0.5f, v2, r2)) | ((uint32_t)f2h(__builtin_fmaf(0.5f, v3, r3)) << 16)};
+                }
         }
         if (t_next >= ntiles) break;
         t = t_next;
+        tile_origin(t, m0, n0);
     }
 }
 
@@ -185,7 +218,7 @@ int launch_sparse24_contract(const uint8_t* data, const uint8_t* meta, const uin
     static std::once_flag once;
     static hipError_t attr = hipSuccess;
     std::call_once(once, [] {
-        attr = hipFuncSetAttribute((const void*)sparse24_contract_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * kSpStage);
+        attr = hipFuncSetAttribute((const void*)sparse24_contract_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kSpStages * kSpStage);
     });
     if (attr != hipSuccess) {
         set_error("hipFuncSetAttribute failed: %s", hipGetErrorString(attr));
@@ -195,7 +228,7 @@ int launch_sparse24_contract(const uint8_t* data, const uint8_t* meta, const uin
     const int tiles = ((m + kBlockM - 1) / kBlockM) * ((n + kBlockN - 1) / kBlockN);
     const int cus = cu_count();
     const int grid = tiles < cus ? tiles : cus - cus % 8;
-    hipLaunchKernelGGL(sparse24_contract_kernel, dim3(grid), dim3(kThreads), 2 * kSpStage, s, a);
+    hipLaunchKernelGGL(sparse24_contract_kernel, dim3(grid), dim3(kThreads), kSpStages * kSpStage, s, a);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
         set_error("sparse contract launch failed: %s", hipGetErrorString(e));

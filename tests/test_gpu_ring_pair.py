@@ -65,3 +65,28 @@ def test_integer_sums(pk):  # noqa: F811
     pk.call("pk_linear_int8_accumulate", a, b, acc, m, n, k)
     ref = a[:m].cpu().numpy().astype(np.int64) @ b.cpu().numpy().astype(np.int64).T
     assert np.array_equal(acc.cpu().numpy(), ref)
+
+
+@pytest.mark.parametrize("m,k", [(16, 128), (272, 256), (528, 384), (16400, 512), (8208, 4096)])
+def test_sparse_contract_stages(pk, m, k):  # noqa: F811
+    """The sparse contract's three-stage ring across tiles: one to four K-steps
+    (fewer than stages, and not a multiple of them), several tiles a workgroup,
+    ragged rows.  Exact inputs (0, +-1 activations, +-2^i weights, scales a power
+    of two), so the fp16 result is known: max|err| = 0."""
+    g = torch.Generator(device="cuda")
+    g.manual_seed(m + k)
+    dense = torch.zeros((m, k // 4, 4), device="cuda")
+    pos = torch.randint(0, 3, (m, k // 4), generator=g, device="cuda")
+    first, second = pos, torch.full_like(pos, 3)
+    val = torch.randint(-1, 2, (2, m, k // 4), generator=g, device="cuda").float()
+    dense.scatter_(2, first[..., None], val[0][..., None]).scatter_(2, second[..., None], val[1][..., None])
+    codes = val.permute(1, 2, 0).reshape(m, k // 2).to(torch.float8_e4m3fn).view(torch.uint8)
+    nib = (first | (second << 2)).to(torch.uint8)
+    meta = (nib[:, 0::2] | (nib[:, 1::2] << 4)).contiguous()
+    buf = torch.cat([codes.reshape(-1), meta.reshape(-1)])
+    w = torch.randint(-2, 3, (1024, k), generator=g, device="cuda").float()
+    scales = torch.full((1024,), 0.125, device="cuda")
+    out = torch.randint(-8, 9, (m, 1024), generator=g, device="cuda").half()
+    want = out.double() + 0.5 * (dense.reshape(m, k).double() @ w.double().t()) * 0.125 / 16.0
+    pk.call("pk_ffn_contract_fp8_sparse", buf, w.to(torch.float8_e4m3fn).view(torch.uint8), scales, out, m, k)
+    assert torch.equal(out, want.half())
