@@ -469,7 +469,9 @@ int32_t pk_gemm_k_split(int32_t format, int32_t epilogue, int32_t m, int32_t n, 
 /* Batch-1 joint GEMV for `steps` consecutive frames:
  *   score[o] = bias[o] + w_scale[o] * sum_k W[o,k] * relu(enc[t,k] + pred[k])
  * for o < outputs, then decision[2t] = argmax over the first token_outputs
- * scores (ties to the lower id) and decision[2t+1] = the duration argmax over
+ * scores (ties to the lower id; a NaN score never wins, and a frame whose token
+ * scores are all NaN is token 0, here and in the scan and the decoders) and
+ * decision[2t+1] = the duration argmax over
  * the next `durations` scores (first maximum wins).  weight is fp16
  * (weight_int8 = 0, w_scales ignored, may be NULL) or int8 with per-row fp32
  * scales.  enc is fp16 [steps x enc_stride], pred fp32 [hidden]; scores

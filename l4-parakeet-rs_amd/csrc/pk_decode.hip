@@ -39,6 +39,7 @@
 // state stays in the owning wave's registers, layer 0's in every thread that
 // evaluates the unit; the INT8 layer-1 banks, the candidate fp32 layer-1
 // output, the layer-0 sums and the prediction go through the workspace.
+#include "pk_decision.hpp"
 #include "pk_kernels.hpp"
 
 namespace pk {
@@ -704,7 +705,7 @@ __global__ __launch_bounds__(kDecThreads, 1) void tdt_decode_kernel(DecodeArgs p
             if (tid < kWin) {
                 unsigned long long b = win_w[0][tid];
                 for (int i = 1; i < 4; ++i) b = win_w[i][tid] > b ? win_w[i][tid] : b;
-                win_tok[tid] = (int)(0xffffu - (((uint32_t)b) >> 16));
+                win_tok[tid] = key_token((uint32_t)b);
             }
             __syncthreads();
             // the greedy rules (decoder.cu:773-783) over the window, identical in
@@ -960,7 +961,7 @@ __global__ __launch_bounds__(k640Threads) void tdt_decode_640_kernel(DecodeArgs 
     };
     auto decisions = [&]() {
         const u64 b = max8(win_s[lane >> 3][lane & 7]);
-        return (int)(0xffffu - ((uint32_t)b >> 16)) | (win_dur[lane & 7] << 16);
+        return key_token((uint32_t)b) | (win_dur[lane & 7] << 16);
     };
 
     // ---- wave 10: the encoder rows ---------------------------------------------

@@ -5,6 +5,7 @@
 // fp16 per pass, the activation vector staged once per block in LDS.
 #include <mutex>
 
+#include "pk_decision.hpp"
 #include "pk_kernels.hpp"
 
 namespace pk {
@@ -379,7 +380,7 @@ __global__ __launch_bounds__(256, 2) void joint_scan_kernel(ScanArgs p) {
 #pragma unroll
             for (int off = 1; off < 64; off <<= 1) best = max_level(best, off);
             if (lane == 0) {
-                dec_tok[wave + 4 * h] = (int)(0xffffu - (((uint32_t)best) >> 16));
+                dec_tok[wave + 4 * h] = key_token((uint32_t)best);
                 dec_dur[wave + 4 * h] = dur;
             }
         }
