@@ -39,6 +39,7 @@
 // state stays in the owning wave's registers, layer 0's in every thread that
 // evaluates the unit; the INT8 layer-1 banks, the candidate fp32 layer-1
 // output, the layer-0 sums and the prediction go through the workspace.
+#include "pk_cell.hpp"
 #include "pk_decision.hpp"
 #include "pk_kernels.hpp"
 
@@ -111,53 +112,6 @@ __device__ __forceinline__ float wave_max(float v) {
 
 // decoder.cu:95-97 quantize_i8: round to nearest even, clamp to +-127.
 __device__ __forceinline__ int quant_i8(float v) { return max(-127, min(127, (int)__builtin_rintf(v))); }
-
-// exp(x) from IEEE basic operations only, so that the long form's cell (whose
-// outputs are rounded to INT8) is reproduced bit for bit by a CPU evaluating
-// the same operations: Cody-Waite reduction x = n ln2 + r (ln2 split into a
-// 16-bit head, so n * head is exact, and a tail), e^r by its degree-7 Taylor
-// polynomial (|r| <= 0.347: truncation error 5e-9 relative), times 2^n.
-// Within 0.82 ulp of exp over [-87, 88]; expf / tanhf of the reference are
-// within about an ulp too.
-__device__ __forceinline__ float det_exp(float x) {
-    if (x != x) return x;
-    x = __builtin_fminf(__builtin_fmaxf(x, -104.0f), 89.0f);
-    const float n = __builtin_rintf(x * 1.44269504f);
-    float r = __builtin_fmaf(n, -0.693145751953125f, x);
-    r = __builtin_fmaf(n, -1.428606765330187e-06f, r);
-    float q = 1.98412698e-04f;
-    q = __builtin_fmaf(q, r, 1.38888889e-03f);
-    q = __builtin_fmaf(q, r, 8.33333333e-03f);
-    q = __builtin_fmaf(q, r, 4.16666667e-02f);
-    q = __builtin_fmaf(q, r, 1.66666667e-01f);
-    q = __builtin_fmaf(q, r, 0.5f);
-    q = __builtin_fmaf(q, r, 1.0f);
-    q = __builtin_fmaf(q, r, 1.0f);
-    return __builtin_ldexpf(q, (int)n);
-}
-// The IEEE quotient 1 / s for s >= 1 (or NaN).  Below 2^96 it is one Newton
-// step on the hardware reciprocal: compared with the division for every
-// mantissa (the step scales with powers of two), no bit differs; three
-// instructions instead of the division's ten.
-__device__ __forceinline__ float rcp_rn(float s) {
-    if (__builtin_amdgcn_ballot_w64(!(s < 0x1p96f)) != 0) return 1.0f / s;
-    const float r = __builtin_amdgcn_rcpf(s);
-    return __builtin_fmaf(__builtin_fmaf(-r, s, 1.0f), r, r);
-}
-__device__ __forceinline__ float det_sigmoid(float v) { return rcp_rn(1.0f + det_exp(-v)); }
-// tanh(x) = sign(x) (1 - e^-2|x|) / (1 + e^-2|x|): absolute error ~1e-7.
-__device__ __forceinline__ float det_tanh(float v) {
-    const float t = det_exp(-2.0f * __builtin_fabsf(v));
-    return __builtin_copysignf(div_rn(1.0f - t, 1.0f + t, rcp_rn(1.0f + t)), v);
-}
-
-// decoder.cu:116-129 lstm_cell with the transcendental functions above; the
-// cell update is fma(f, c, i * g).
-__device__ __forceinline__ void lstm_cell(const float (&s)[4], float c_prev, float& c_out, float& h_out) {
-    const float ig = det_sigmoid(s[0]), fg = det_sigmoid(s[1]), cg = det_tanh(s[2]), og = det_sigmoid(s[3]);
-    c_out = __builtin_fmaf(fg, c_prev, ig * cg);
-    h_out = og * det_tanh(c_out);
-}
 
 __device__ __forceinline__ uint32_t ld_word(const uint32_t* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 __device__ __forceinline__ void st_word(uint32_t* p, uint32_t v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
@@ -1250,10 +1204,7 @@ __global__ __launch_bounds__(k640Threads) void tdt_decode_640_kernel(DecodeArgs 
                 const int sum = half_row_isum((hi ? ra : ia) + dpp_mov<0x128>(hi ? ia : ra));
                 if ((lane & 15) == 8) r0_s[wave * 4 + gate] = sum;  // wave 10 publishes them
                 const float v = __builtin_fmaf((float)sum, cq[2], __builtin_fmaf((float)rs, cq[1], bias1));
-                // det_sigmoid, or det_tanh for the cell gate, with one exponential
-                const float e = det_exp(gate == 2 ? -2.0f * __builtin_fabsf(v) : -v);
-                const float r = rcp_rn(1.0f + e);
-                const int act = __float_as_int(gate == 2 ? __builtin_copysignf(div_rn(1.0f - e, 1.0f + e, r), v) : r);
+                const int act = __float_as_int(det_gate(v, gate == 2));
                 const float ig = __int_as_float(__builtin_amdgcn_readlane(act, 0)), fg = __int_as_float(__builtin_amdgcn_readlane(act, 16));
                 const float cg = __int_as_float(__builtin_amdgcn_readlane(act, 32)), og = __int_as_float(__builtin_amdgcn_readlane(act, 48));
                 c_new[1] = __builtin_fmaf(fg, c_cur[1], ig * cg);
