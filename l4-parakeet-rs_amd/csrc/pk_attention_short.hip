@@ -5,14 +5,15 @@
 // per-head position packer of the cached position projections
 // (encoder.cu:1321-1336, encoder.rs:442-480).
 //
-// Short attention of up to 128 rows (longer ones: pk_attention_tile.hpp): one
-// wave64 per (query, head).  Scores: the 64 lanes form
+// Short attention of few rows or narrow windows (short_takes_tile; the others:
+// pk_attention_tile.hpp): one wave64 per (query, head).  Scores: the 64 lanes form
 // four 16-lane groups, each lane holding 8 of the head's 128 dimensions as one
 // 16-byte load of K and of the packed position row, so one pass scores four
 // keys; a 16-lane DPP row sum gives each key's score, scaled by 1/sqrt(128)
 // and kept in the wave's LDS row.  Softmax over the <= 257 scores with the
 // wave's max and sum, then the context: lane l accumulates dimensions 2l and
 // 2l+1 over the keys, probability = exp(s - max) / sum, as the reference.
+#include "pk_attention_rule.hpp"
 #include "pk_attention_tile.hpp"
 #include "pk_kernels.hpp"
 
@@ -202,11 +203,8 @@ void launch_pack_position_heads(const uint16_t* in, uint16_t* out, hipStream_t s
 void launch_local_attention_short(const uint16_t* q, const uint16_t* k, const uint16_t* v, const uint16_t* pos,
                                   const uint16_t* bu, const uint16_t* bv, uint16_t* out, int rows, int padded_rows,
                                   int valid_rows, int left, int right, hipStream_t s) {
-    // One wave per (query, head) while its at most 128 keys are few rounds of
-    // loads; longer windows on the fp32 tile kernel, whose queries share the
-    // rows (measured: 48 rows 5.4 against 9.2 us, 96 rows 8.5 / 11.6, 144 rows
-    // 13.6 / 13.9, 300 rows 25.0 / 19.4, 496 rows 34.2 / 21.4).
-    if (padded_rows <= 128) {
+    const int live = min(min(rows, valid_rows), padded_rows);
+    if (!short_takes_tile(live, min(valid_rows, left + right + 1), cu_count())) {
         ShortArgs a{q, k, v, pos, bu, bv, out, rows, padded_rows, valid_rows, left, right};
         attention_short_kernel<<<dim3((padded_rows + 3) / 4, kHeadsN), 256, 0, s>>>(a);
         return;

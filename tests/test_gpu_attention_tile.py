@@ -1,8 +1,8 @@
-"""The fp32 attention tile kernel at the edges of its tiles, against the oracle:
-the short form past 128 rows (ragged last tiles, windows narrower than the model's,
-fewer valid rows than rows), and values that are not finite, which may reach only the
-queries whose window holds them (oracle run on the finite values for the others).
-Bar: max|err| <= 1e-2 * RMS(oracle), that of the short form's other tests."""
+"""The short form past 128 rows at the edges of its kernels' tiles, against the oracle
+(ragged last tiles, windows narrower than the model's, fewer valid rows than rows, on
+the wave kernel and on the fp32 tile kernel), and values that are not finite, which may
+reach only the queries whose window holds them (oracle run on the finite values for the
+others).  Bar: max|err| <= 1e-2 * RMS(oracle), that of the short form's other tests."""
 import numpy as np
 import pytest
 
@@ -74,3 +74,32 @@ def test_value_quantizer_row_sizes(pk, orc, rows, edge):  # noqa: F811
     for f, r in np.argwhere(np.isnan(vt)):
         ref[el + (f * rows + r) // 2] &= 0x0F if r & 1 else 0xF0
     np.testing.assert_array_equal(host(out), ref)
+
+
+@pytest.mark.parametrize("padded,rows,valid,left,right", [
+    (400, 399, 390, 95, 3), (512, 512, 500, 0, 128), (448, 447, 440, 60, 37), (352, 352, 352, 128, 0), (529, 529, 529, 128, 70),
+    (1024, 1024, 1023, 101, 19)])
+def test_tile_narrow_windows(pk, orc, padded, rows, valid, left, right):  # noqa: F811
+    """Windows narrower than the model's in calls that take the tile kernel."""
+    test_tile_edges(pk, orc, padded, rows, valid, left, right)
+
+
+@pytest.mark.parametrize("bad", [np.nan, np.inf])
+def test_tile_non_finite_values_short_form(pk, orc, bad):  # noqa: F811
+    """As test_tile_non_finite_values, in a call that takes the tile kernel."""
+    padded, left, right = 416, 70, 40
+    q, k, v, pos, bu, bv = inputs(78, padded)
+    spoilt = v.copy()
+    for at in (0, 200, 415):
+        spoilt[at, 5::7] = bad
+    got = run(pk, (q, k, spoilt, pos, bu, bv), padded, padded, padded, left, right).astype(np.float64)
+    ref = orc.local_attention_short(q, k, v, pos, bu, bv, padded, valid_rows=padded, left=left, right=right).astype(np.float64)
+    sees = np.zeros(padded, bool)
+    for at in (0, 200, 415):
+        sees |= (np.arange(padded) - left <= at) & (at <= np.arange(padded) + right)
+    hit = np.zeros(1024, bool)
+    hit[5::7] = True
+    clean = ~(sees[:, None] & hit[None, :])
+    assert not np.isfinite(got[~clean]).any()
+    assert np.isfinite(got[clean]).all()
+    assert np.abs(got - ref)[clean].max() <= TOL * np.sqrt((ref ** 2).mean())
