@@ -168,18 +168,23 @@ def _stream(stream=None):
     return raw(torch.cuda.current_device())
 
 
-# name -> (function, per argument before the stream: is it a pointer)
+# name -> (function, per argument before the stream: is it a pointer), for the
+# entry points whose last argument can be a stream
 _ENTRIES = {name: (getattr(lib, name), tuple(t is P for t in args[:-1]))
             for name, (res, args) in SIGNATURES.items() if args and args[-1] is P}
 
 
 def call(name: str, *args, stream=None) -> None:
     """Call `name` with tensors converted to device pointers; raise on error."""
-    fn, pointers = _ENTRIES[name]
-    if len(args) != len(pointers):
-        raise TypeError(f"{name} takes {len(pointers)} arguments and the stream, got {len(args)}")
-    status = fn(*[a.data_ptr() if p and a is not None and not isinstance(a, int) else a for a, p in zip(args, pointers)],
-                _stream(stream))
+    fn, pointers = _ENTRIES.get(name, (None, ()))
+    if fn is not None and len(args) == len(pointers):
+        conv = [a.data_ptr() if p and a is not None and not isinstance(a, int) else a for a, p in zip(args, pointers)]
+    else:
+        # an entry point without a stream, or all arguments given (what follows
+        # them is not read), or too few, which ctypes refuses
+        fn = getattr(lib, name)
+        conv = [_ptr(a) if t is P else a for a, t in zip(args, fn.argtypes)]
+    status = fn(*conv, _stream(stream))
     if status < 0:
         raise PkError(f"{name}: status {status}: {last_error()}")
 
