@@ -179,10 +179,15 @@ static bool has_ring(int fmt, int epi) {
 template <int F> static int ring_stages_of(int kAI) {
     return kAI == 1 ? g3::LS<F, 1>::kS : (kAI == 2 ? g3::LS<F, 2>::kS : (kAI == 3 ? g3::LS<F, 3>::kS : g3::LS<F, 4>::kS));
 }
+// FP8 and INT8 on 32 and 64 rows: those of the pair kernel (K a multiple of 256;
+// other K run the plain ring, one stage shorter on 32 rows, as long on 64).
+template <int F> static int byte_ring_stages(int kAI) {
+    return kAI == 1 ? 2 * g3::LP<F, 1>::kPairs : (kAI == 2 ? 2 * g3::LP<F, 2>::kPairs : ring_stages_of<F>(kAI));
+}
 static int ring_stages(int fmt, int kAI) {
     switch (fmt) {
-    case FMT_FP8: return ring_stages_of<FMT_FP8>(kAI);
-    case FMT_I8: return ring_stages_of<FMT_I8>(kAI);
+    case FMT_FP8: return byte_ring_stages<FMT_FP8>(kAI);
+    case FMT_I8: return byte_ring_stages<FMT_I8>(kAI);
     case FMT_G128A8: return ring_stages_of<FMT_G128A8>(kAI);
     default: return ring_stages_of<FMT_G128A16>(kAI);
     }

@@ -137,6 +137,22 @@ def test_gemm_tile_plan(lib):
     assert _tile(lib, 99, EPI_F16, 16, 256)[0] == -4
 
 
+@pytest.mark.skipif(os.environ.get("PK_GEMM_TILE_ROWS") is not None, reason="tile size forced")
+def test_gemm_tile_pair_stages(lib):
+    """FP8, INT8 and GLU tiles of 32 and 64 rows hold pairs of stages: four pairs of
+    20 KiB stages, three of 24 KiB; 128 rows the plain ring's four of 32 KiB."""
+    FP8, I8 = 0, 1
+    EPI_F16, EPI_F32, EPI_GLU = 0, 3, 6
+    for fmt in (FP8, I8):
+        assert _tile(lib, fmt, EPI_F16, 96, 1024) == (32, 128, 8)
+        assert _tile(lib, fmt, EPI_F32, 496, 4096) == (64, 128, 6)
+        assert _tile(lib, fmt, EPI_F16, 750, 4096) == (128, 128, 4)
+    assert _tile(lib, FP8, EPI_GLU, 96, 2048) == (32, 128, 8)
+    assert _tile(lib, FP8, EPI_GLU, 752, 2048) == (64, 128, 6)
+    assert _tile(lib, FP8, EPI_GLU, 1500, 2048) == (128, 128, 4)
+    assert _tile(lib, FP8, EPI_GLU, 7504, 2048) == (256, 256, 2)
+
+
 def test_gemm_k_split(lib):
     """The K split over a ring workgroup's waves: INT4-g128 formats on 32-row
     ring tiles with k >= 1024 only (the T = 750 FF2 of BASELINE config 3)."""
