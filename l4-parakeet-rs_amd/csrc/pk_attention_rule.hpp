@@ -1,5 +1,5 @@
-// Which kernel a short-form attention call takes.  constexpr, so that the same
-// function runs in a host test.
+// Which kernel a short-form attention call takes, and the rows a tile of the
+// tile kernel loads.  constexpr, so that the same functions run in a host test.
 #pragma once
 
 namespace pk {
@@ -21,5 +21,16 @@ constexpr bool short_takes_tile(int live, int keys, int cus) {
     const bool full = 3 * (long long)tiles >= (3LL * rounds - 1) * cus;
     return keys >= (full ? 96 : (rounds <= 1 ? 160 : 192));
 }
+
+// A tile of 16 queries from qb < live loads whole blocks of rows, more than its
+// queries see: rows past their last key (or before key 0) are those at the
+// ends instead, and queries without an output the last live one.  K and V may
+// end there: valid_rows may exceed padded_rows, and the window's right end the rows of K.
+constexpr int tile_last_key(int qb, int live, int valid, int right) {
+    const int reach = (qb + 15 < live - 1 ? qb + 15 : live - 1) + right;
+    return reach < valid - 1 ? reach : valid - 1;
+}
+constexpr int tile_key_row(int key, int last_key) { return key < 0 ? 0 : (key < last_key ? key : last_key); }
+constexpr int tile_query_row(int query, int live) { return query < live - 1 ? query : live - 1; }
 
 }  // namespace pk

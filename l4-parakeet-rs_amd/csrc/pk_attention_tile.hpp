@@ -24,6 +24,7 @@
 
 #include <float.h>
 
+#include "pk_attention_rule.hpp"
 #include "pk_common.hpp"
 
 namespace pk {
@@ -66,6 +67,7 @@ __global__ __launch_bounds__(kTileThreads, 2) void attention_tile_kernel(Attenti
     // a wave's LDS accesses complete in order; the compiler must not move them
     auto wave_order = []() { asm volatile("" ::: "memory"); };
     if (qb < live_end) {
+        const int last_key = tile_last_key(qb, live_end, p.valid_rows, p.right);
         // ---- values of features 32 (wave % 4) + 2 l16, + 1: the first four waves take
         // key columns 0 .. 143, the others 144 .. 271, lane group g columns 16 t + 4 g ..
         const int feature = 32 * (wave & 3) + 2 * l16, half = wave >> 2;
@@ -83,7 +85,7 @@ __global__ __launch_bounds__(kTileThreads, 2) void attention_tile_kernel(Attenti
                 const int i = min(lane + 64 * k, v_chunks - 1), r = v_row(i), c = v_col(i);
                 const uint8_t* src;
                 if constexpr (kMode == kTileShort) {
-                    const int key = min(max(first_key + 144 * half + r, 0), p.valid_rows - 1);
+                    const int key = tile_key_row(first_key + 144 * half + r, last_key);
                     src = (const uint8_t*)p.value + ((size_t)key * kModel + head * kHead + 32 * (wave & 3)) * 2 + 16 * c;
                 } else {
                     const int key = min(max(first_key + 144 * half + 16 * c, 0), p.value_stride - 16);
@@ -105,13 +107,13 @@ __global__ __launch_bounds__(kTileThreads, 2) void attention_tile_kernel(Attenti
             }
         };
         // ---- scores: four waves content, four position, every fourth block of 16 columns
-        const int c_lo = max(0, -first_key), c_hi = min(p.valid_rows - 1, qb + 15 + p.right) - first_key;
+        const int c_lo = max(0, -first_key), c_hi = last_key - first_key;
         const int which = wave >> 2;
         const int b_lo = (which == 0 ? c_lo : max(0, c_lo - 15)) >> 4;
         const int b_hi = (which == 0 ? c_hi : min(p.left + p.right, c_hi)) >> 4;
         float a[32];
         {
-            const uint16_t* q = p.query + (size_t)min(qb + l16, p.padded_rows - 1) * kModel + head * kHead + 32 * g;
+            const uint16_t* q = p.query + (size_t)tile_query_row(qb + l16, live_end) * kModel + head * kHead + 32 * g;
             const uint16_t* u = (which == 0 ? p.bias_u : p.bias_v) + head * kHead + 32 * g;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
@@ -129,7 +131,7 @@ __global__ __launch_bounds__(kTileThreads, 2) void attention_tile_kernel(Attenti
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int col = 16 * b + 4 * i + g;
-                const uint16_t* src = which == 0 ? p.key + (size_t)min(max(first_key + col, 0), p.valid_rows - 1) * kModel + head * kHead
+                const uint16_t* src = which == 0 ? p.key + (size_t)tile_key_row(first_key + col, last_key) * kModel + head * kHead
                                                  : p.position + ((size_t)head * kPosRows + min(col, kPosRows - 1)) * kHead;
                 r[i] = ((const v4i*)src)[l16];
             }
@@ -213,7 +215,7 @@ __global__ __launch_bounds__(kTileThreads, 2) void attention_tile_kernel(Attenti
             }
         };
         // this lane's two features at columns at .. at + 3 of its half, 0 for keys
-        // outside [0, valid_rows) (whose e4m3 bytes the quantizer does not write)
+        // outside [0, last_key] (past valid_rows the quantizer does not write the e4m3 bytes)
         auto values4 = [&](int at, float (&y0)[4], float (&y1)[4]) {
             uint32_t v0 = 0, v1 = 0;
             if constexpr (kMode != kTileShort) {
@@ -223,7 +225,7 @@ __global__ __launch_bounds__(kTileThreads, 2) void attention_tile_kernel(Attenti
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int key = first_key + 144 * half + at + i;
-                const bool in = key >= 0 && key < p.valid_rows;
+                const bool in = key >= 0 && key <= last_key;
                 constexpr float kValueScale = 8.0f / 448.0f;  // V holds v * 56
                 float a, b;
                 if constexpr (kMode == kTileShort) {

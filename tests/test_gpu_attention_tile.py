@@ -103,3 +103,43 @@ def test_tile_non_finite_values_short_form(pk, orc, bad):  # noqa: F811
     assert not np.isfinite(got[~clean]).any()
     assert np.isfinite(got[clean]).all()
     assert np.abs(got - ref)[clean].max() <= TOL * np.sqrt((ref ** 2).mean())
+
+
+@pytest.mark.parametrize("rows,valid,right", [(496, 600, 0), (490, 600, 0), (496, 500, 2), (512, 4096, 0)])
+def test_tile_keys_end_with_the_window(pk, orc, rows, valid, right):  # noqa: F811
+    """valid_rows past the rows of Q, K and V, which end with the last key of the last
+    query's window."""
+    left, keys = 128, min(valid, rows + right)
+    q, k, v, pos, bu, bv = inputs(500 + rows + right, keys)
+    got = run(pk, (q[:rows], k, v, pos, bu, bv), rows, rows, valid, left, right)
+    ref = orc.local_attention_short(q, k, v, pos, bu, bv, rows, valid_rows=keys, left=left, right=right)
+    g, r = got.astype(np.float64), ref[:rows].astype(np.float64)
+    assert np.abs(g - r).max() <= TOL * np.sqrt((r ** 2).mean())
+
+
+@pytest.mark.parametrize("rows,at", [(752, 3), (752, 750), (4000, 100), (4000, 3990), (15008, 40)])
+def test_boundary_tiles_non_finite_values(pk, orc, rows, at):  # noqa: F811
+    """NaN bytes of the long form's e4m3 V (the tc form) in a boundary tile's keys
+    reach the queries whose window holds them and no others of the boundary."""
+    q, k, v, pos, bu, bv = inputs(600 + at, rows)
+    value = torch.empty((1024, rows), dtype=torch.uint8, device="cuda")
+    pk.call("pk_quantize_fp8_fixed_transpose", dev(v), value, rows, 56.0)
+    outs = []
+    for spoil in (False, True):
+        if spoil:
+            value[5::7, at] = 0x7F
+        out = torch.empty((rows, 1024), dtype=torch.int16, device="cuda")
+        pk.call("pk_local_relpos_attention_tc_scores", dev(q), dev(k), dev(v), value, dev(pos), dev(bu), dev(bv), out, rows, rows, rows,
+                128, 128, rows)
+        outs.append(host(out).view(np.float16).astype(np.float64))
+    clean_run, got = outs
+    hit = np.zeros(1024, bool)
+    hit[5::7] = True
+    sees = np.abs(np.arange(rows) - at) <= 128
+    # queries of the fp32 boundary tiles: below the first whole window, past the last
+    edge = (np.arange(rows) < 128) | (np.arange(rows) >= 16 * ((rows - 144) // 16 + 1))
+    assert np.isnan(got[np.ix_(sees & edge, hit)]).all()
+    other = edge[:, None] & ~(sees[:, None] & hit[None, :])
+    assert np.isfinite(got[other]).all()
+    # the same sums in another order (fp32), rounded to fp16
+    assert np.abs(got - clean_run)[other].max() <= 2 ** -10 * np.abs(clean_run[other]).max()
