@@ -57,6 +57,20 @@ def test_glu_small_grids(pk, m, valid):  # noqa: F811
     assert not small[valid:m].any() and bool((small[m] == 77).all())
 
 
+@pytest.mark.parametrize("m,k", [(1, 640), (96, 128), (96, 640), (250, 384), (500, 640), (752, 1152), (1500, 640)])
+def test_glu_odd_steps(pk, m, k):  # noqa: F811
+    """GLU through pk_gemm with K an odd multiple of 128: the plain ring on 32-row
+    tiles, the two-waves-per-SIMD ring on 64- and 128-row ones."""
+    n, glu = 2048, 6
+    assert pk.gemm_tile(0, glu, m, n)[0] in (32, 64, 128)
+    a, b, rs, ws = operands(0, m, n, k)
+    small = torch.full((m + 1, n // 2), 77, dtype=torch.float16, device="cuda")
+    large = torch.zeros((LARGE, n // 2), dtype=torch.float16, device="cuda")
+    pk.gemm(0, glu, a, b, m, n, k, small, w_scales=ws, row_scales=rs, ldo=n // 2)
+    pk.gemm(0, glu, a, b, LARGE, n, k, large, w_scales=ws, row_scales=rs, ldo=n // 2)
+    assert torch.equal(small[:m], large[:m]) and bool((small[m] == 77).all()) and bool(small[:m].any())
+
+
 def test_integer_sums(pk):  # noqa: F811
     """INT8 through the pairs against exact integer products."""
     m, n, k = 70, 256, 1024
