@@ -566,8 +566,8 @@ int32_t pk_tdt_decode_long(const uint16_t* enc, int32_t frames, int32_t enc_stri
  * written by pk_quantize_value_int4{,_register} with value_stride =
  * padded_rows: FP8 V [1024 x stride] (v * 56), S4 V [1024 x stride / 2],
  * 1024 float per-feature scales.  Tiles of 16 queries whose window lies in
- * [0, valid_rows) take the quantized tile path; all other queries the FP32
- * per-query path; rows >= min(rows, valid_rows) are written as zero.
+ * [0, valid_rows) take the quantized tile path; the other tiles the FP32 path
+ * (fp32 MFMA sums); rows >= min(rows, valid_rows) are written as zero.
  * Requirements: padded_rows % 16 == 0, rows and valid_rows in (0, padded_rows],
  * value_stride >= padded_rows and % 16 == 0, attention_left = attention_right
  * = 128, 16-byte aligned operands.  `value` (fp16 V) is not read. */
@@ -586,7 +586,7 @@ int32_t pk_quantize_value_int4(const uint16_t* input, uint8_t* output, int32_t e
                                void* stream);
 /* encoder.cu:597-634 pk_sm89_quantize_value_int4_register: as above, but FP8 V
  * is written only for row pairs (2i, 2i+1) with 2i < 272 or 2i + 1 >=
- * valid_rows - 272 (the keys the per-query boundary path reads). */
+ * valid_rows - 272 (the keys whose FP8 V the FP32 boundary tiles use). */
 int32_t pk_quantize_value_int4_register(const uint16_t* input, uint8_t* output, int32_t elements,
                                         float inverse_scale, int32_t valid_rows, void* stream);
 /* encoder.cu:2024-2036 pk_sm89_local_relpos_attention_tc_scores: fp16 scores,
@@ -615,7 +615,8 @@ int32_t pk_local_relpos_attention_packed(const uint16_t* query, const uint16_t* 
  * 1024], packed position table [8 x 272 x 128] (pk_pack_position_heads), fp32
  * scores (q + u).k + (q + v).p over 128 dimensions times 1/sqrt(128), softmax,
  * fp16 output [padded_rows x 1024]; rows at or beyond min(rows, valid_rows)
- * are zero.  attention_left, attention_right <= 128. */
+ * are zero.  attention_left, attention_right <= 128.  valid_rows may exceed
+ * padded_rows: K and V then hold the rows up to the last key that a query sees. */
 int32_t pk_local_relpos_attention(const uint16_t* query, const uint16_t* key, const uint16_t* value,
                                   const uint16_t* position, const uint16_t* bias_u, const uint16_t* bias_v,
                                   uint16_t* output, int32_t rows, int32_t padded_rows, int32_t valid_rows,

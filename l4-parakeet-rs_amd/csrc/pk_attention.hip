@@ -864,8 +864,8 @@ int launch_pack_vectors(bool int4, const uint16_t* in, uint8_t* out, float* scal
 
 int launch_quantize_value_int4(const uint16_t* vt, uint8_t* out, int rows, float inverse_scale, bool edge_only, int valid_rows,
                                hipStream_t s) {
-    // by what a thread holds: 2, 4 or 8 chunks of 8 keys (256 threads: 16384
-    // rows), then 1024 threads (65536 rows, two workgroups a CU)
+    // by what a thread holds: 1, 4 or 8 chunks of 8 keys (256 threads: 16384
+    // rows), then 4, 6 or 8 of 1024 threads (65536 rows, two workgroups a CU)
     const int chunks = (rows + 7) / 8;
 #define PK_VALUE_REG(threads, per) \
     quantize_value_reg_kernel<threads, per><<<kModel, threads, 0, s>>>(vt, out, rows, inverse_scale, edge_only ? 1 : 0, valid_rows)

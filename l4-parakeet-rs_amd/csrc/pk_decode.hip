@@ -730,10 +730,14 @@ __global__ __launch_bounds__(kDecThreads, 1) void tdt_decode_kernel(DecodeArgs p
 //    1, 2, 4, ..., 32, but N sums reduced together halve their number at each
 //    level (lanes_sum): 16 sums take about 60 instructions instead of 200.
 // Every sum has the association of tdt_decode_kernel's, so the tokens are the same.
-// 7500 frames, 2333 tokens, INT8 joint, long form: 41.1 -> 19.6 ms (8.2 us a
-// token: three exchanges of 0.8 us, 0.9 us for layer 0 and 0.8 us each for the
-// joint and for layer 1); on a slower box 69.3 -> 31.7 ms.  93 frames, fp16
-// form: 1003 -> 600 us on the latter.
+// 7500 frames, INT8 joint, long form: 41.1 -> 19.6 ms; on a slower box 69.3 ->
+// 31.7 ms.  93 frames, fp16 form: 1003 -> 600 us on the latter.  Where a token's
+// time goes (long form, 7500 frames, 2513 updates and 2520 joint rounds in 21.1
+// ms, 8.4 us each, by cycle stamps in workgroup 0, which cost 2 % of it): layer
+// 0 with the wait for its sums 1.5 us, layer 1 0.4 and its exchange 2.0, the
+// projection 0.2 and its exchange 0.9, the joint 1.6 and its exchange 1.5, the
+// greedy rules 0.3.  An exchange ends with the slowest workgroup, hence more than
+// the 1.31 us it takes by itself, or less where work runs under it.
 constexpr int k640H = 640, k640KP = 5, k640Blocks = 64, k640Waves = 10, k640Rows = 16;
 constexpr int k640Threads = 64 * (k640Waves + 1);  // and a wave that loads the encoder rows
 constexpr int k640Ring = 32;                        // encoder rows kept in LDS
@@ -1100,7 +1104,9 @@ __global__ __launch_bounds__(k640Threads) void tdt_decode_640_kernel(DecodeArgs 
     float c_cur[2] = {0.0f, 0.0f}, c_new[2] = {0.0f, 0.0f};         // cell states of unit u
     while (g.frame < p.frames) {
         // Packed weights are unpacked where they are used: without this the
-        // compiler hoists the conversions out of the loop and spills.
+        // compiler hoists the conversions out of the loop and spills.  The
+        // fp16 form still spills a few of the 168 registers that eleven waves
+        // leave (6 with an INT8 joint, 9 with an fp16 one); the long form none.
         auto keep = [](uint32_t& w) { asm volatile("" : "+v"(w)); };
 #pragma unroll
         for (int j = 0; j < KP; ++j) {

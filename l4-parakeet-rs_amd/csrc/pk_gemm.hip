@@ -379,7 +379,8 @@ static int by_epi(int epi, const GemmArgs& a, hipStream_t s) {
         if constexpr (F == FMT_I8 || F == FMT_S4 || F == FMT_I8_SKIP) return launch_fmt<F, EPI_I32>(a, s);
         break;
     case EPI_GLU:
-        // the paired value / gate weight rows need the 256-column tiles
+        // glu_row pairs value and gate weight rows within 16 rows, so tiles of 128 weight
+        // rows serve as well as 256
         if constexpr (F == FMT_FP8) {
             if (a.n % 256 != 0 || a.ldo != a.n / 2 || !a.w_scales) {
                 set_error("GLU needs n %% 256 == 0 weight rows, ldo == n/2 and weight scales");

@@ -1,4 +1,4 @@
-// Occupancy-2 GEMM engine (gfx950) for every format but the GLU epilogue.
+// Occupancy-2 GEMM engine (gfx950) for every format (GLU on its one-tile rings only).
 //
 // Two independent workgroups share each CU, so one workgroup's epilogue
 // (VALU: scaling, SiLU, conversions, stores) and its barrier waits run while
@@ -938,8 +938,6 @@ __global__ __launch_bounds__(kThreads, 1) void gemm3_ring_pair_kernel(GemmArgs p
     }
 }
 
-// ---- small grids, long K: one 32 x 128 tile per workgroup, K split over its 4 waves ----
-//
 // The ring kernel with two waves per SIMD: waves w and w + 4 share quadrant
 // w % 4 of the tile (its 64 columns and 16 kAI rows) and take its first
 // ceil(kAI / 2) / remaining row blocks, so each SIMD runs two independent
@@ -1068,6 +1066,8 @@ __global__ __launch_bounds__(2 * kThreads, 1) void gemm3_ring8_kernel(GemmArgs p
     }
 }
 
+// ---- small grids, long K: one 32 x 128 tile per workgroup, K split over its 4 waves ----
+//
 // For the group-wise INT4 formats at small T (FF2 at T = 750: 192 tiles of
 // 32 rows, K = 4096) the ring kernel above is a chain of K-steps whose every
 // link is an LDS read, the INT4 decode and the MFMAs; the tile count cannot

@@ -1,18 +1,18 @@
 """GPU parity of the long-form local attention path (encoder.cu:561-634,
 :1476-2097) against the CPU oracle, through the C ABI.
 
-Packers and the value quantizer are integer/byte work: bit-exact.  The
-attention outputs follow the reference operation by operation; the only
-arithmetic the GPU and the oracle do not share is the softmax exponential
-(host libm expf in the oracle; in the packed and tc kernels the hardware's
-approximate exponential, as the reference's --use_fast_math build has it,
-within a few ulp; in the boundary path the device expf), which can move a U4
-probability or an output rounding by one step.  The packed kernel's e4m3 bytes must therefore be equal
-except for at most 0.1 % of them, which may differ by one code.  The tc
-kernel's fp16 outputs: its fp32 score sums run in the MFMA's order (as on
-the reference's tensor cores, unspecified), so an e4m3 probability that lies
-within an ulp of a rounding boundary can round to the neighbouring code; the
-query's context for that head then moves by that step times the key's V row.
+Packers and the value quantizer are integer/byte work: bit-exact. The interior
+tiles of the packed form follow the reference operation by operation but for
+the softmax exponential (host libm expf in the oracle, the hardware's
+approximate exponential in the kernels, as the reference's --use_fast_math
+build has it, within a few ulp), which can move a U4 probability or an output
+rounding by one step; the boundary tiles sum in fp32 in the MFMA's order, which
+can move an output rounding too. The packed kernel's e4m3 bytes must therefore
+be equal except for at most 0.1 % of them, which may differ by one code. The tc
+kernel's fp16 outputs: its fp32 score sums run in the MFMA's order (as on the
+reference's tensor cores, unspecified), so an e4m3 probability that lies within
+an ulp of a rounding boundary can round to the neighbouring code; the query's
+context for that head then moves by that step times the key's V row.
 The bar: every (query, head) block within max|err| <= 1e-2 * RMS(oracle
 output), except at most 0.1 % of blocks whose deviation is such a step at one
 or two keys (after removing it, the block is within the same bar).
