@@ -3,8 +3,7 @@
 One step = every encoder linear of all 24 layers (FF1 expand/contract, QKV,
 attention out, pointwise1, pointwise2, FF2 expand/contract) on the MI355X
 kernels, each layer's linears in a seeded mix of FP8 / INT8 / INT4-g128
-formats.  Inputs and packed weights are resident in
-HBM before timing; weights are random-init with the real shapes (no
+formats.  Inputs and packed weights are resident in HBM before timing; weights are random-init with the real shapes (no
 checkpoint is available), activations are synthetic.  Prints one JSON line.
 """
 import argparse
@@ -924,7 +923,7 @@ def joint_bench(pk, torch, stream, reps=2000):
 
 
 def decode_bench(pk, torch, stream, frames=45000):
-    """BASELINE configs[4]'s decoder: batch-1 greedy TDT decode of T frames in
+    """The stack's decoder: batch-1 greedy TDT decode of T frames in
     one persistent launch (2-layer LSTM, 640 hidden; INT8 joint 640 -> 1030),
     synthetic random weights and encoder rows, the joint bias favouring the
     blank and duration 1 so tokens come about every 5 frames, roughly the rate
@@ -1097,7 +1096,7 @@ def roof(flops, nbytes, peak_tops):
 
 
 def config_results(pk, torch, stream, reps=10):
-    """BASELINE configs 1-4 on the GPU: per GEMM TOPS, GB/s (algorithmic bytes)
+    """The four single-layer workloads on the GPU: per GEMM TOPS, GB/s (algorithmic bytes)
     and the fraction of its roofline min(MFMA peak, AI x 8 TB/s) (5.0 PF for
     FP8 / INT8 MFMAs, 2.5 PF for the fp16 MFMAs of the INT4-g128 x fp16
     kernels, which also report the 5.0 PF fraction), from the average
@@ -1161,7 +1160,7 @@ def config_results(pk, torch, stream, reps=10):
     def rows_q(kind, t, k, src=None, outliers=False):
         if src is None:
             x = torch.randn((t, k), generator=g, device=dev)
-            if outliers:  # 0.1 % of the entries at +-20, seeded positions
+            if outliers:  # FP8 layer: 0.1 % of the entries at +-20, seeded positions
                 mask = torch.rand((t, k), generator=g, device=dev) < 1e-3
                 sign = torch.where(torch.rand((t, k), generator=g, device=dev) < 0.5, -20.0, 20.0)
                 x = torch.where(mask, sign, x)
@@ -1401,7 +1400,7 @@ def main():
     ap.add_argument("--only-producers", action="store_true", help="run only the activation producers' timing")
     ap.add_argument("--hipblaslt", action="store_true",
                     help="yardstick: hipBLASLt (torch._scaled_mm) against this library's FP8 kernels on the stack's shapes")
-    ap.add_argument("--only-configs", action="store_true", help="run only the BASELINE config 1-4 measurements")
+    ap.add_argument("--only-configs", action="store_true", help="run only the single-layer workloads")
     ap.add_argument("--only-clock", action="store_true",
                     help="run only the shader-clock probe (FF1 expand FP8 with random vs all-zero operands)")
     ap.add_argument("--only-refplan", action="store_true",
@@ -1535,7 +1534,7 @@ def main():
                    "format_plan_seed": "0x5EED0005", "parallelism": "none (1 GPU)"},
         "pct_mfma_peak": round(100.0 * tops / PEAK["fp8"], 2),
         "ms_per_audio_min": round(ms_step / audio_min, 4),
-        # BASELINE config 5 by part, each measured above in this run at T=45000 (60 min of audio):
+        # ms per audio minute by part, each measured above in this run at T=45000 (60 min of audio):
         # the linear stack, 24 layers of packed local attention with its packers, the greedy decode
         "config5_ms_per_audio_min": {
             "linear_stack": round(ms_step / audio_min, 4),

@@ -146,7 +146,7 @@ int32_t pk_pack_int8_rows(const uint16_t* weight, int32_t n, int32_t k, int8_t* 
  * byte j = q[2j] & 15 | q[2j+1] << 4; packed is [n x k/2]. */
 int32_t pk_pack_int4_rows(const uint16_t* weight, int32_t n, int32_t k, uint8_t* packed, float* scales,
                           void* stream);
-/* No reference counterpart (BASELINE config 3): group-wise asymmetric INT4,
+/* No reference counterpart: group-wise asymmetric INT4,
  * 128-K groups, q packed 8 per uint32 ([n x k/8]), fp16 scales and integer
  * fp16 zero-points ([n x k/128]); dequant (q - z) * s. */
 int32_t pk_pack_int4_g128(const uint16_t* weight, int32_t n, int32_t k, uint32_t* packed,
@@ -279,7 +279,7 @@ int32_t pk_linear_fp8_dyn(const uint8_t* input, const float* input_scales, const
  * operands packed two per byte ([m x k/2], [n x k/2]). */
 int32_t pk_linear_int4_accumulate(const uint8_t* input, const uint8_t* weight_oi, int32_t* accumulators,
                                   int32_t m, int32_t n, int32_t k, void* stream);
-/* No reference counterpart (BASELINE config 3).  fp16 activations x
+/* No reference counterpart.  fp16 activations x
  * group-wise INT4 weights (pk_pack_int4_g128 layout), weights dequantized to
  * fp16 in registers, fp32 accumulate; bias may be NULL; fp16 or fp32 output. */
 int32_t pk_linear_int4g128(const uint16_t* input, const uint32_t* weight_q, const uint16_t* weight_scales,
@@ -374,7 +374,7 @@ int32_t pk_subsample_pointwise_fp8(const uint8_t* input, const uint8_t* weight, 
                                    const float* input_scales, const float* bias, uint16_t* output, int32_t rows,
                                    void* stream);
 
-/* Activation-sparse FF2 contract (BASELINE config 4; the reference's sparse
+/* Activation-sparse FF2 contract (the reference's sparse
  * FF2 is the 2:4 path, encoder.cu:1087-1095): INT8 activations [rows x 4096]
  * with per-row scales (zeros where the frame's activations were dropped) x
  * per-row INT8 weights [1024 x 4096] -> fp32 [rows x 1024],
@@ -386,7 +386,7 @@ int32_t pk_ffn_contract_int8_rowskip(const int8_t* input, const float* input_sca
                                      const float* weight_scales, float* output, int32_t rows, uint32_t* skip_counts,
                                      void* stream);
 
-/* Exact 2:4 form of the activation-sparse FF2 (BASELINE config 4).  The
+/* Exact 2:4 form of the activation-sparse FF2.  The
  * reference's sparse FF2 (encoder.cu:685-704 selection, :1037-1095 contract)
  * keeps the two largest magnitudes of every quartet and drops the rest; here
  * the dropped nonzeros are kept in a per-row overflow list, so the contract

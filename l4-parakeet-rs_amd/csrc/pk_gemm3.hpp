@@ -657,7 +657,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm3_kernel(GemmArgs p) {
 
 // ---- small grids: one tile per workgroup, an S-stage ring -----------------
 //
-// When a launch has no more tiles than CUs (INT4-g128 at
+// When a launch has no more tiles than CUs (INT8 750 x 1024 -> 4096, INT4-g128 at
 // T = 750), every workgroup computes exactly one tile and the K-loop is the
 // whole latency chain: with the engine's one-step prefetch each K-step waits
 // for a memory round trip.  This variant gives the one workgroup of a CU an

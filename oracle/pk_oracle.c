@@ -573,7 +573,7 @@ void orc_quantize_fp8_rows(const uint16_t* x, int rows, int valid_rows, int k, u
     }
 }
 
-/* Dynamic per-token INT8 (BASELINE config 3 "mixed variant"; no reference
+/* Dynamic per-token INT8 (INT4-g128 FF, mixed variant; no reference
  * counterpart, pinned by closed form): scale = max|x| / 127 (1 if zero),
  * q = clamp(rne(x / scale), +-127). */
 void orc_quantize_int8_rows(const uint16_t* x, int rows, int valid_rows, int k, int8_t* q,
@@ -785,8 +785,8 @@ void orc_compress_24(const uint8_t* x, int rows, int k, uint8_t* data, uint8_t* 
     }
 }
 
-/* Exact 2:4 form of INT8 rows (the activation-sparse FF2 of BASELINE config
- * 4): per quartet the selection of orc_compress_24 on int8 magnitudes |v|
+/* Exact 2:4 form of INT8 rows (the activation-sparse FF2, per-frame
+ * top-k): per quartet the selection of orc_compress_24 on int8 magnitudes |v|
  * (encoder.cu:685-704 keeps the two largest, ties to the lower index, in index
  * order), and every nonzero it drops goes to the row's overflow list as
  * (element << 8) | byte in ascending element order.  counts[r] entries at

@@ -103,7 +103,7 @@ def _tile(lib, fmt, epi, m, n):
 @pytest.mark.skipif(os.environ.get("PK_GEMM_TILE_ROWS") is not None, reason="tile size forced")
 def test_gemm_tile_plan(lib):
     """The launcher's tile choice on a 256-CU part (the host-only fallback
-    when no GPU is visible, and MI355X's count): the BASELINE sizes the
+    when no GPU is visible, and MI355X's count): the sizes the
     full-size parity tests use reach the 256-row kernels; grids of at most
     one tile per CU take the one-tile-per-workgroup ring (more stages)."""
     FP8, I8, G128A8, F16, G128A16, I8SKIP, Q4K = 0, 1, 3, 4, 5, 6, 7
@@ -121,7 +121,7 @@ def test_gemm_tile_plan(lib):
     assert _tile(lib, I8SKIP, EPI_F32, 7500, 1024) == (128, 128, 2)
     assert _tile(lib, F16, EPI_F16, 45000, 1024) == (256, 256, 2)
     assert _tile(lib, Q4K, EPI_F16, 16, 256) == (256, 256, 2)
-    # small grids: BASELINE config 1 (750 x 4096) in 128-row ring tiles,
+    # small grids: INT8 750 x 4096 in 128-row ring tiles,
     # the T = 750 INT4-g128 FF2 (750 x 1024) in 32-row ring tiles
     rows, cols, stages = _tile(lib, I8, EPI_F32, 750, 4096)
     assert (rows, cols) == (128, 128) and stages >= 3
@@ -155,7 +155,7 @@ def test_gemm_tile_pair_stages(lib):
 
 def test_gemm_k_split(lib):
     """The K split over a ring workgroup's waves: INT4-g128 formats on 32-row
-    ring tiles with k >= 1024 only (the T = 750 FF2 of BASELINE config 3)."""
+    ring tiles with k >= 1024 only (the T = 750 FF2)."""
     I8, G128A8, G128A16 = 1, 3, 5
     EPI_F16, EPI_F8, EPI_F32 = 0, 1, 3
     ks = lib.pk_gemm_k_split

@@ -1,5 +1,5 @@
-"""Full-size parity: the GEMM kernel variants the benchmark times, at the
-BASELINE sizes, against the CPU oracle on sampled rows.
+"""Full-size parity: the GEMM kernel variants the benchmark times, at its
+sizes, against the CPU oracle on sampled rows.
 
 The launcher picks the tile height from the grid (pk_gemm_tile reports it),
 so small test shapes never reach the 256-row kernels that run the T = 7500 /
@@ -126,7 +126,7 @@ def pack(pk, fmt, n, k, gen):
 
 
 def activations(pk, t, k, kind, gen, outliers=True):
-    """fp16 ~N(0,1) with 0.1 % outliers at +-20 (BASELINE config 2), quantized
+    """fp16 ~N(0,1) with 0.1 % outliers at +-20, quantized
     per row on the GPU (kind 0 FP8, 1 INT8); the quantizer is pinned bit-exact
     elsewhere, and only its output is used here."""
     x = torch.randn((t, k), generator=gen, device="cuda")
@@ -216,7 +216,7 @@ class Layer:
         return rows_tile
 
 
-# ---- BASELINE config 2: one FP8 layer at T = 7500 ----------------------------------
+# ---- one FP8 layer at T = 7500 ----------------------------------
 
 def test_c2_fp8_layer_T7500(pk, orc):
     """QKV (fp16), attention out (+residual), FF1 (e4m3 SiLU), FF2 (+0.5
@@ -231,7 +231,7 @@ def test_c2_fp8_layer_T7500(pk, orc):
             assert layer.check(name, n, k, epi) == want[name], name
 
 
-# ---- BASELINE config 5: one stack layer at T = 45000 in each format ----------------
+# ---- one stack layer at T = 45000 in each format ----------------
 
 @pytest.mark.parametrize("fmt", ["fp8", "int8", "int4g128"])
 def test_stack_layer_T45000(pk, orc, fmt):
@@ -245,7 +245,7 @@ def test_stack_layer_T45000(pk, orc, fmt):
     torch.cuda.empty_cache()
 
 
-# ---- BASELINE config 3: INT4-g128 FF1 / FF2 at T = 7500 and 45000 --------------------
+# ---- INT4-g128 FF1 / FF2 at T = 7500 and 45000 --------------------
 
 @pytest.mark.parametrize("t", [7500, 45000])
 def test_c3_int4g128_full(pk, orc, t):
@@ -275,7 +275,7 @@ def test_c3_int4g128_full(pk, orc, t):
     torch.cuda.empty_cache()
 
 
-# ---- BASELINE config 4: activation-sparse FF2 at T = 7500 ----------------------------
+# ---- activation-sparse FF2 at T = 7500 ----------------------------
 
 @pytest.mark.parametrize("sparsity", [0.5, 0.8, 0.9, 0.95])
 def test_c4_rowskip_T7500(pk, orc, sparsity):

@@ -2,7 +2,7 @@
 
 Integer, byte and index results are compared bit-exactly; fp32-accumulated
 FP8 / FP16 / INT4-g128 outputs within max|err| <= 1e-2 * RMS(reference output),
-the tolerance BASELINE.json's north star states.  All calls go through the
+the library's stated tolerance.  All calls go through the
 C ABI (parakeet_linear is a ctypes mirror of include/pk_linear.h).
 """
 import sys
@@ -263,7 +263,7 @@ def test_int8_accumulators_exact(pk, orc, m, n, k):
 
 
 def test_int8_linear_epilogue_config1(pk, orc):
-    """BASELINE config 1: W[4096x1024] ~N(0,0.02) -> per-row INT8, x[750x1024]."""
+    """W[4096x1024] ~N(0,0.02) -> per-row INT8, x[750x1024]."""
     note("int8 linear config 1")
     m, n, k = 750, 4096, 1024
     w = weights(n, k, 0x5EED0001)

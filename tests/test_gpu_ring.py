@@ -1,5 +1,5 @@
 """Parity of the one-tile-per-workgroup ring GEMM (grids of at most one tile
-per CU: BASELINE config 1, the T = 750 INT4-g128 linears) against the CPU
+per CU: INT8 750 x 1024 -> 4096, the T = 750 INT4-g128 linears) against the CPU
 oracle, through the C ABI: INT8 accumulators and INT4-g128 x INT8 outputs
 bit for bit, FP8 / INT4-g128 x fp16 outputs within 1e-2 x RMS.  Shapes cover
 a single K-step, fewer K-steps than ring stages, many more, and ragged M."""
@@ -78,7 +78,7 @@ def test_ring_int8_accumulators_exact(pk, orc, m, n, k):
 
 
 def test_ring_int8_dyn_config1(pk, orc):
-    """BASELINE config 1's GEMM (750 x 1024 -> 4096, per-token INT8, fp32 out)."""
+    """The small INT8 GEMM (750 x 1024 -> 4096, per-token INT8, fp32 out)."""
     m, n, k = 750, 4096, 1024
     ring(pk, pk.FMT_I8, pk.EPI_F32, m, n)
     rng = np.random.default_rng(0x5EED0001)

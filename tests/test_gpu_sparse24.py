@@ -1,4 +1,4 @@
-"""Exact 2:4 activation-sparse FF2 (BASELINE config 4) against the oracle.
+"""Exact 2:4 activation-sparse FF2 against the oracle.
 
 The producer (pk_quantize_rows_int8_sparse24) must give the INT8 bytes and
 scales of the dense per-row quantizer, the reference's 2:4 selection of them
